@@ -89,6 +89,24 @@ def test_draws_reproducible_and_seed_dependent(qf):
     assert np.mean(a != c) > 0.9
 
 
+@pytest.mark.parametrize("n", [1, 3, 6, 7, 10, 11, 20, 21, 23])
+@pytest.mark.parametrize("zeros", [False, True])
+def test_many_draws_continue_few(qf, n, zeros):
+    # draw t depends on (state, seed, t) alone: a call of many draws (segment
+    # table) starts with the draws of a call of few (one wave a draw); 21 and
+    # 23 qubits have 2 and 8 scan segments, 65 more draws a partial last block
+    psi = _random_state(n, 50 + n)
+    if zeros:
+        psi[(np.arange(psi.size) % 7) > 1] = 0
+        psi[psi.size // 2:psi.size // 2 + psi.size // 4] = 0
+        psi[0] = 0.5
+    d = _dev(qf, psi)
+    few = qf.backend.evaluate(qf.backend.sample_indices(d, 1000, 9))
+    many = qf.backend.evaluate(qf.backend.sample_indices(d, 4096 + 65, 9))
+    np.testing.assert_array_equal(many[:1000], few)
+    assert np.all(np.abs(psi[many]) > 0)
+
+
 def test_empty_and_invalid(qf):
     psi = _dev(qf, _random_state(4, 1))
     assert qf.backend.sample_indices(psi, 0, 1).numel() == 0
