@@ -442,6 +442,14 @@ int qfx_qaoa_status(const void* sync, int* failed);
 int qfx_mlp_gemm(void* stream, void* C, const void* A, const void* B, int M,
                  int N, int K, int64_t sam, int64_t sak, int64_t sbk,
                  int64_t sbn, const void* bias /*[N] or NULL*/, int relu);
+/* The same, then C *= (mask > 0) where mask [M x N] is given (the input
+ * gradient masked by the ReLU of the layer below), and where rowsum [M] is
+ * given rowsum[m] = sum_k A(m, k) (the bias gradient, of a weight-gradient
+ * product). */
+int qfx_mlp_gemm_fused(void* stream, void* C, const void* A, const void* B,
+                       int M, int N, int K, int64_t sam, int64_t sak,
+                       int64_t sbk, int64_t sbn, const void* bias, int relu,
+                       const void* mask, void* rowsum);
 /* dz = dy * (y > 0) */
 int qfx_mlp_relu_bwd(void* stream, void* dz, const void* dy, const void* y,
                      int64_t len);

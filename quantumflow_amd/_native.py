@@ -81,6 +81,8 @@ SIGNATURES = {
     'qfx_qaoa_run': (_i, [_vp, _vp]),
     'qfx_qaoa_status': (_i, [_vp, _vp]),
     'qfx_mlp_gemm': (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i64, _i64, _i64, _vp, _i]),
+    'qfx_mlp_gemm_fused': (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i64, _i64, _i64, _vp, _i,
+                                _vp, _vp]),
     'qfx_mlp_relu_bwd': (_i, [_vp, _vp, _vp, _vp, _i64]),
     'qfx_mlp_colsum': (_i, [_vp, _vp, _vp, _i, _i]),
     'qfx_mlp_mse_workspace': (_i64, [_i64]),

@@ -87,10 +87,12 @@ class AngleProposer:
 
     # ---- kernels --------------------------------------------------------
     def _gemm(self, C, A, B, M, N, K, sam, sak, sbk, sbn, bias=None, relu=False,
-              boff=0, bias_off=0, aoff=0, coff=0):
-        _native.call('qfx_mlp_gemm', bk.stream_handle(), _vp(C, coff), _vp(A, aoff),
+              boff=0, bias_off=0, aoff=0, coff=0, mask=None, rowsum=None, rowsum_off=0):
+        _native.call('qfx_mlp_gemm_fused', bk.stream_handle(), _vp(C, coff), _vp(A, aoff),
                      _vp(B, boff), M, N, K, sam, sak, sbk, sbn,
-                     None if bias is None else _vp(bias, bias_off), int(relu))
+                     None if bias is None else _vp(bias, bias_off), int(relu),
+                     None if mask is None else _vp(mask),
+                     None if rowsum is None else _vp(rowsum, rowsum_off))
 
     def forward(self, x, keep=False):
         """x: [B, 19] float32 device tensor -> [B, 2p] (and the activations)."""
@@ -110,22 +112,18 @@ class AngleProposer:
     def backward(self, acts, dy):
         """Parameter gradients into self.grads for d loss / d output = dy."""
         B = dy.shape[0]
-        s = bk.stream_handle()
-        g = dy.contiguous()
+        g = dy.contiguous()                      # d loss / d (pre-activation) of layer li
         for li in reversed(range(len(self.layout))):
             wo, bo, fi, fo = self.layout[li]
             x = acts[li]
-            if li < len(self.layout) - 1:
-                dz = torch.empty_like(g)
-                _native.call('qfx_mlp_relu_bwd', s, _vp(dz), _vp(g), _vp(acts[li + 1]), g.numel())
-                g = dz
             # dW = dz^T x ; db = column sums of dz
-            self._gemm(self.grads, g, x, fo, fi, B, 1, fo, fi, 1, coff=wo)
-            _native.call('qfx_mlp_colsum', s, _vp(self.grads, bo), _vp(g), B, fo)
+            self._gemm(self.grads, g, x, fo, fi, B, 1, fo, fi, 1, coff=wo,
+                       rowsum=self.grads, rowsum_off=bo)
             if li > 0:
-                dx = torch.empty(B, fi, dtype=torch.float32, device=g.device)
-                self._gemm(dx, g, self.params, B, fi, fo, fo, 1, fi, 1, boff=wo)
-                g = dx
+                # the layer below ends in a ReLU: its output x masks the gradient
+                dz = torch.empty(B, fi, dtype=torch.float32, device=g.device)
+                self._gemm(dz, g, self.params, B, fi, fo, fo, 1, fi, 1, boff=wo, mask=x)
+                g = dz
 
     def loss_and_grad(self, x, t):
         """MSE loss (0-dim device tensor) and gradients in self.grads."""

@@ -50,6 +50,46 @@ def test_forward_and_gradients_vs_oracle(P):
         assert np.max(np.abs(gb - db)) <= 1e-4 * (1 + np.max(np.abs(db)))
 
 
+@pytest.mark.parametrize("M_,N_,K_", [(1, 1, 1), (1, 8, 19), (31, 33, 7), (32, 32, 8),
+                                      (33, 31, 256), (64, 96, 257), (256, 19, 512), (70, 40, 1031)])
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("off", [0, 1])
+def test_gemm_forms(P, M_, N_, K_, ta, tb, off):
+    # edges of the 32 x 32 tile, of the 8-wide k blocks and their 8-wave
+    # batches, both orders of each operand, aligned and unaligned bases
+    import torch
+    from quantumflow_amd import _native, backend as bk
+    rng = np.random.default_rng(M_ + 3 * N_ + 5 * K_)
+    a = rng.normal(size=(M_, K_)).astype(np.float32)
+    b = rng.normal(size=(K_, N_)).astype(np.float32)
+    bias = rng.normal(size=N_).astype(np.float32)
+    mask = rng.normal(size=(M_, N_)).astype(np.float32)
+
+    def put(m, transposed):
+        flat = np.concatenate([np.zeros(off, np.float32), (m.T if transposed else m).reshape(-1)])
+        return torch.from_numpy(flat).cuda(), P._vp
+    (da, vp), (db, _) = put(a, ta), put(b, tb)
+    dbias, dmask = torch.from_numpy(bias).cuda(), torch.from_numpy(mask).cuda()
+    c = torch.full((M_ * N_ + 1,), 7.0, dtype=torch.float32, device='cuda')
+    rs = torch.full((M_ + 1,), 7.0, dtype=torch.float32, device='cuda')
+    sa = (1, M_) if ta else (K_, 1)
+    sb = (1, K_) if tb else (N_, 1)
+    _native.call('qfx_mlp_gemm_fused', bk.stream_handle(), vp(c), vp(da, off), vp(db, off), M_, N_,
+                 K_, sa[0], sa[1], sb[0], sb[1], vp(dbias), 1, vp(dmask), vp(rs))
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    want = np.maximum(a64 @ b64 + bias, 0) * (mask > 0)
+    # sums of K + 1 terms: at most (K + 8) roundings of 2^-24, each of the
+    # terms' absolute sum
+    tol = (K_ + 8) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64) + np.abs(bias))
+    got = c.cpu().numpy().astype(np.float64)
+    assert np.all(np.abs(got[:-1].reshape(M_, N_) - want) <= tol)
+    assert got[-1] == 7.0
+    r = rs.cpu().numpy().astype(np.float64)
+    assert np.all(np.abs(r[:-1] - a64.sum(1)) <= (K_ + 8) * 2.0 ** -24 * np.abs(a64).sum(1))
+    assert r[-1] == 7.0
+
+
 def test_adam_vs_oracle(P):
     prop = P.AngleProposer(p=2, hidden=(16,), seed=4)
     rng = np.random.default_rng(1)
