@@ -95,6 +95,29 @@ def test_permutation_gates_exact(bk, name, k):
         assert np.array_equal(got, ref), (name, axes)
 
 
+@pytest.mark.parametrize("n", [3, 6, 12])
+@pytest.mark.parametrize("name,params,k", [('RX', (0.7,), 1), ('X', (), 1), ('T', (), 1),
+                                           ('CNOT', (), 2), ('XX', (0.3,), 2), ('CCNOT', (), 3)])
+def test_gates_around_the_line_bits(bk, n, name, params, k):
+    # lowest target on either side of bit 3 (a 128-byte line), in and out of place
+    import itertools
+    rng = np.random.default_rng(31 + n)
+    psi = rand_state(n, rng)
+    m = O.gate_matrix(name, *params)
+    kind = bk.classify(m)
+    src = bk.as_device(bk.astensorproduct(psi))
+    for bits in itertools.permutations(range(min(n, 5)), k):
+        axes = [n - 1 - b for b in bits]
+        ref = O.tensormul(m.reshape([2] * (2 * k)), psi, axes)
+        got = gpu_tensormul(bk, m, psi, axes)
+        work = src.clone()
+        bk.apply_gate(work, work, n, list(bits), kind, inplace_sparse=True)
+        if name in ('X', 'CNOT', 'CCNOT'):
+            assert np.array_equal(got, ref), bits
+        assert np.max(np.abs(got - ref)) <= TOL, bits
+        assert np.array_equal(bk.evaluate(work).reshape(ref.shape), got), bits
+
+
 def test_inplace_sparse_matches_out_of_place(bk):
     import torch
     rng = np.random.default_rng(13)
