@@ -103,6 +103,13 @@ int64_t qfx_reduce_workspace_bytes(int64_t len);
 /* result[0] = sum_i conj(a_i) b_i   (np.vdot), complex128 in device memory */
 int qfx_inner(void* stream, void* result, const void* a, const void* b,
               int64_t len, void* workspace);
+/* result[0] = sum_i conj(a_i) b_j, where bit src_bit[b] of j equals bit b of
+ * i: qfx_inner with qfx_permute_qubits(b), without storing the permuted b.
+ * 10 <= n.  src_bit: host, a permutation of 0..n-1.  workspace:
+ * qfx_reduce_workspace_bytes(2^n). */
+int qfx_inner_permuted(void* stream, void* result, const void* a,
+                       const void* b, int n, const int* src_bit,
+                       void* workspace);
 /* out[i] = |in_i| (hypot), float64 */
 int qfx_abs(void* stream, void* out, const void* in, int64_t len);
 /* out[i] = |in_i|^2, float64 */

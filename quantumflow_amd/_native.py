@@ -55,6 +55,7 @@ SIGNATURES = {
     'qfx_apply_monomial_inplace': (_i, [_vp, _vp, _i, _i, _ip, _ip, _cp]),
     'qfx_reduce_workspace_bytes': (_i64, [_i64]),
     'qfx_inner': (_i, [_vp, _vp, _vp, _vp, _i64, _vp]),
+    'qfx_inner_permuted': (_i, [_vp, _vp, _vp, _vp, _i, _ip, _vp]),
     'qfx_abs': (_i, [_vp, _vp, _vp, _i64]),
     'qfx_abs2': (_i, [_vp, _vp, _vp, _i64]),
     'qfx_expect_diag': (_i, [_vp, _vp, _vp, _vp, _i64, _vp]),

@@ -53,6 +53,9 @@ EINSUM_SUBSCRIPTS = string.ascii_lowercase + string.ascii_uppercase
 pi = np.pi
 
 _NP_CTYPE = np.complex128
+# smallest state qfx_inner_permuted takes (index bits of its tile)
+_PERM_TILE_BITS = 10
+
 _inited = set()
 _props = {}
 _workspace = {}
@@ -447,6 +450,27 @@ def inner(tensor0: BKTensor, tensor1: BKTensor) -> BKTensor:
     res = torch.empty((), dtype=CTYPE, device=a.device)
     ws = workspace(_native.load().qfx_reduce_workspace_bytes(a.numel()))
     _native.call('qfx_inner', stream_handle(), _ptr(res), _ptr(a), _ptr(b), a.numel(), _ptr(ws))
+    return res
+
+
+def inner_permuted(tensor0: BKTensor, tensor1: BKTensor, src_bit: typing.List[int]) -> BKTensor:
+    """inner(tensor0, tensor1 with its index bits relabelled): bit src_bit[b]
+    of tensor1's index is bit b of tensor0's.  One pass over both; the
+    relabelled tensor is written only where it is smaller than a tile."""
+    a = as_device(tensor0)
+    b = as_device(tensor1)
+    if a.numel() != b.numel():
+        raise ValueError('inner: tensors differ in size')
+    n = len(src_bit)
+    bits = _native.int_array(src_bit)
+    if n < _PERM_TILE_BITS:
+        c = torch.empty_like(b)
+        _native.call('qfx_permute_qubits', stream_handle(), _ptr(c), _ptr(b), n, bits)
+        return inner(a, c)
+    res = torch.empty((), dtype=CTYPE, device=a.device)
+    ws = workspace(_native.load().qfx_reduce_workspace_bytes(a.numel()))
+    _native.call('qfx_inner_permuted', stream_handle(), _ptr(res), _ptr(a), _ptr(b), n, bits,
+                 _ptr(ws))
     return res
 
 

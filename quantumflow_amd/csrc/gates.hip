@@ -12,6 +12,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "permute_tile.h"
 #include "qfx_common.h"
 
 namespace {
@@ -157,7 +158,33 @@ __global__ __launch_bounds__(kBlock) void dense_dev_kernel(double2* __restrict__
 }
 
 // out[i] = in[j] where bit src[b] of j equals bit b of i (a relabelling of
-// the index bits; writes are coalesced, reads gather).
+// the index bits), by tiles that read and write contiguous runs.
+// 26 qubits, 2 GiB moved: a random order 415 us (5.2 TB/s), the reversed order
+// 401 us; by gathering 1096 and 2122 us.
+__global__ __launch_bounds__(kPermBlock) void permute_tile_kernel(double2* __restrict__ out,
+                                                                 const double2* __restrict__ in,
+                                                                 uint64_t ntiles, PermTile p) {
+  __shared__ v2d lds[1 << kPermT];
+  const PermLane q = perm_lane(p);
+  for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    uint64_t bi, bo;
+    perm_bases(p, tile, &bi, &bo);
+    v2d v[kPermPer];
+    const v2d* src = reinterpret_cast<const v2d*>(in) + bi + q.in_lane;
+#pragma unroll
+    for (int u = 0; u < kPermPer; ++u) v[u] = ld_stream(src + q.in_u[u]);
+#pragma unroll
+    for (int u = 0; u < kPermPer; ++u) lds[q.lds_in[u]] = v[u];
+    __syncthreads();
+    v2d* dst = reinterpret_cast<v2d*>(out) + bo + q.out_lane;
+#pragma unroll
+    for (int u = 0; u < kPermPer; ++u)
+      st_stream(dst + q.out_u[u], lds[perm_swz(threadIdx.x + kPermBlock * u)]);
+    __syncthreads();
+  }
+}
+
+// The same for states smaller than a tile.
 struct PermArg {
   int src[QFX_MAX_QUBITS];
 };
@@ -341,16 +368,19 @@ int qfx_permute_qubits(void* stream, void* out, const void* in, int n, const int
   if (out == in) return qfx::set_error(QFX_EINVAL, "qfx_permute_qubits: out must not alias in");
   if (n < 1 || n > QFX_MAX_QUBITS)
     return qfx::set_error(QFX_ERANGE, "qfx_permute_qubits: n out of range");
+  int rc = qfx::check_permutation(n, src_bit, "qfx_permute_qubits");
+  if (rc) return rc;
+  const uint64_t len = (uint64_t)1 << n;
+  if (n >= kPermT) {
+    const uint64_t ntiles = len >> kPermT;
+    hipLaunchKernelGGL(permute_tile_kernel, dim3((unsigned)(ntiles < (1u << 20) ? ntiles : 1u << 20)),
+                       dim3(kPermBlock), 0, qfx::as_stream(stream), static_cast<double2*>(out),
+                       static_cast<const double2*>(in), ntiles, make_perm_tile(n, src_bit));
+    return qfx::check_launch("permute_tile_kernel");
+  }
   PermArg a;
   std::memset(&a, 0, sizeof(a));
-  uint64_t seen = 0;
-  for (int b = 0; b < n; ++b) {
-    if (src_bit[b] < 0 || src_bit[b] >= n || ((seen >> src_bit[b]) & 1))
-      return qfx::set_error(QFX_EINVAL, "qfx_permute_qubits: not a permutation");
-    seen |= (uint64_t)1 << src_bit[b];
-    a.src[b] = src_bit[b];
-  }
-  const uint64_t len = (uint64_t)1 << n;
+  for (int b = 0; b < n; ++b) a.src[b] = src_bit[b];
   hipLaunchKernelGGL(permute_bits_kernel, dim3((unsigned)((len + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, qfx::as_stream(stream), static_cast<double2*>(out),
                      static_cast<const double2*>(in), len, n, a);

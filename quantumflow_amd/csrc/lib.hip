@@ -38,6 +38,16 @@ int check_targets(int n, int k, const int* targets, int kmax, const char* fn) {
   return QFX_OK;
 }
 
+int check_permutation(int n, const int* src_bit, const char* fn) {
+  uint64_t seen = 0;
+  for (int b = 0; b < n; ++b) {
+    if (src_bit[b] < 0 || src_bit[b] >= n || ((seen >> src_bit[b]) & 1))
+      return set_error(QFX_EINVAL, std::string(fn) + ": not a permutation");
+    seen |= (uint64_t)1 << src_bit[b];
+  }
+  return QFX_OK;
+}
+
 void sort_bits(int k, const int* targets, int* sorted) {
   for (int j = 0; j < k; ++j) sorted[j] = targets[j];
   std::sort(sorted, sorted + k);

@@ -21,6 +21,9 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 // Validates a target list: 1 <= k <= kmax, distinct, each < n.
 int check_targets(int n, int k, const int* targets, int kmax, const char* fn);
 
+// Validates that src_bit is a permutation of 0..n-1 (n <= 64).
+int check_permutation(int n, const int* src_bit, const char* fn);
+
 // Host-side: sort k bit positions ascending into `sorted`.
 void sort_bits(int k, const int* targets, int* sorted);
 

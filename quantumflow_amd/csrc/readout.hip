@@ -10,13 +10,14 @@
 #include <mutex>
 #include <string>
 
+#include "permute_tile.h"
 #include "qfx_common.h"
 
 namespace {
 
 constexpr int kBlock = 256;
 constexpr int kMaxRedBlocks = 1024;
-constexpr int kZChunkBits = 16;  // elements per <Z> block = 2^16 (or the whole state)
+constexpr int kZChunkBits = 16;  // most bits of a <Z> block's chunk
 
 // Sum `v` over the block; the result is valid in thread 0.
 template <int NV>
@@ -44,54 +45,85 @@ int red_blocks(uint64_t len) {
 }
 
 // mode 0: sum conj(a) b (complex); 1: sum |a|^2 diag; 2: sum |a|^2
+// Bound by the read.  A block takes kRedPer * 256 consecutive elements at a
+// time, so that the grid walks memory in order (each lane's loads a grid
+// apart instead, a power of two of megabytes, met in the same channels):
+// 26 qubits: norm 207 -> 174 us (6.2 TB/s), inner product 456 -> 345 us.
+constexpr int kRedPer = 4;
+
+template <int MODE>
+__device__ __forceinline__ void red_add(double (&acc)[2], const double2 x, const double2 y) {
+  if (MODE == 0) {
+    acc[0] = fma(x.x, y.x, acc[0]);
+    acc[0] = fma(x.y, y.y, acc[0]);
+    acc[1] = fma(x.x, y.y, acc[1]);
+    acc[1] = fma(-x.y, y.x, acc[1]);
+  } else if (MODE == 1) {
+    acc[0] = fma(fma(x.x, x.x, x.y * x.y), y.x, acc[0]);
+  } else {
+    acc[0] = fma(x.x, x.x, fma(x.y, x.y, acc[0]));
+  }
+}
+
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void reduce_stage1(const double2* __restrict__ a,
                                                        const void* __restrict__ b, uint64_t len,
                                                        double2* __restrict__ partial) {
   __shared__ double lds[2 * 4];
   double acc[2] = {0.0, 0.0};
-  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-  uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-  for (; i + 3 * stride < len; i += 4 * stride) {
-    double2 x[4];
+  auto other = [&](uint64_t i) {
+    if (MODE == 0) return static_cast<const double2*>(b)[i];
+    if (MODE == 1) return make_double2(static_cast<const double*>(b)[i], 0.0);
+    return make_double2(0.0, 0.0);
+  };
+  constexpr uint64_t kStep = kRedPer * kBlock;
+  uint64_t i0 = (uint64_t)blockIdx.x * kStep;
+  for (; i0 + kStep <= len; i0 += (uint64_t)gridDim.x * kStep) {
+    double2 x[kRedPer], y[kRedPer];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) x[u] = a[i + u * stride];
-    if (MODE == 0) {
-      double2 y[4];
+    for (int u = 0; u < kRedPer; ++u) x[u] = a[i0 + threadIdx.x + u * kBlock];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) y[u] = static_cast<const double2*>(b)[i + u * stride];
+    for (int u = 0; u < kRedPer; ++u) y[u] = other(i0 + threadIdx.x + u * kBlock);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        acc[0] = fma(x[u].x, y[u].x, acc[0]);
-        acc[0] = fma(x[u].y, y[u].y, acc[0]);
-        acc[1] = fma(x[u].x, y[u].y, acc[1]);
-        acc[1] = fma(-x[u].y, y[u].x, acc[1]);
-      }
-    } else if (MODE == 1) {
-      double d[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) d[u] = static_cast<const double*>(b)[i + u * stride];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) acc[0] = fma(fma(x[u].x, x[u].x, x[u].y * x[u].y), d[u], acc[0]);
-    } else {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) acc[0] = fma(x[u].x, x[u].x, fma(x[u].y, x[u].y, acc[0]));
-    }
+    for (int u = 0; u < kRedPer; ++u) red_add<MODE>(acc, x[u], y[u]);
   }
-  for (; i < len; i += stride) {
-    const double2 x = a[i];
-    if (MODE == 0) {
-      const double2 y = static_cast<const double2*>(b)[i];
-      acc[0] = fma(x.x, y.x, acc[0]);
-      acc[0] = fma(x.y, y.y, acc[0]);
-      acc[1] = fma(x.x, y.y, acc[1]);
-      acc[1] = fma(-x.y, y.x, acc[1]);
-    } else if (MODE == 1) {
-      const double d = static_cast<const double*>(b)[i];
-      acc[0] = fma(fma(x.x, x.x, x.y * x.y), d, acc[0]);
-    } else {
-      acc[0] = fma(x.x, x.x, fma(x.y, x.y, acc[0]));
+  for (uint64_t i = i0 + threadIdx.x; i < len && i < i0 + kStep; i += kBlock)
+    red_add<MODE>(acc, a[i], other(i));
+  block_sum<2>(acc, lds);
+  if (threadIdx.x == 0) partial[blockIdx.x] = make_double2(acc[0], acc[1]);
+}
+
+// sum conj(a[i]) b[j], bit src[b] of j = bit b of i: the inner product with a
+// state whose qubits are ordered otherwise, without writing that state in the
+// other order.  Tiles of b are read in its own order and turned in LDS, as by
+// permute_tile_kernel.  26 qubits in a random order: 374 us (5.7 TB/s);
+// permuting (415 us) and then multiplying (345 us) moves the state twice more.
+__global__ __launch_bounds__(kPermBlock) void inner_permuted_stage1(
+    const double2* __restrict__ a, const double2* __restrict__ b, uint64_t ntiles,
+    double2* __restrict__ partial, PermTile p) {
+  __shared__ v2d tile_lds[1 << kPermT];
+  __shared__ double lds[2 * 4];
+  double acc[2] = {0.0, 0.0};
+  const PermLane q = perm_lane(p);
+  for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    uint64_t bi, bo;
+    perm_bases(p, tile, &bi, &bo);
+    v2d y[kPermPer];
+    double2 x[kPermPer];
+    const v2d* src = reinterpret_cast<const v2d*>(b) + bi + q.in_lane;
+#pragma unroll
+    for (int u = 0; u < kPermPer; ++u) y[u] = ld_stream(src + q.in_u[u]);
+#pragma unroll
+    for (int u = 0; u < kPermPer; ++u) x[u] = ld_stream(a + bo + q.out_lane + q.out_u[u]);
+#pragma unroll
+    for (int u = 0; u < kPermPer; ++u) tile_lds[q.lds_in[u]] = y[u];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPermPer; ++u) {
+      const v2d z = tile_lds[perm_swz(threadIdx.x + kPermBlock * u)];
+      red_add<0>(acc, x[u], make_double2(z.x, z.y));
     }
+    __syncthreads();
   }
   block_sum<2>(acc, lds);
   if (threadIdx.x == 0) partial[blockIdx.x] = make_double2(acc[0], acc[1]);
@@ -144,8 +176,13 @@ __global__ __launch_bounds__(kBlock) void abs_kernel(double* __restrict__ out,
 
 // <Z> stage 1: block `blk` sums chunk [blk << c, (blk+1) << c).  Element
 // i = base + tid + 256 m; bits 0..7 of i are those of tid, bits 8..c-1 those
-// of m.  Writes partial[blk] = {total, S_0 .. S_{c-1}} with
-// S_b = sum |psi_i|^2 bit_b(i) over the chunk.
+// of m.  Writes column blk of partial ([1 + kZChunkBits][nblk]): the total and
+// S_0 .. S_{c-1}, S_b = sum |psi_i|^2 bit_b(i) over the chunk.  Bound by the
+// read: eight elements a lane in flight, whose three bits of m cost a few adds.
+// 26 qubits 180 us, 5.9 TB/s (256 us with one load in flight); 20 qubits 20 us with both stages against 73 us, when its
+// 16 chunks of 2^16 left the chip idle.
+constexpr int kZPer = 8;
+
 __global__ __launch_bounds__(kBlock) void z_stage1(const double2* __restrict__ psi, int c,
                                                   double* __restrict__ partial) {
   __shared__ double lds[(1 + 8 + 8) * 4];
@@ -155,15 +192,26 @@ __global__ __launch_bounds__(kBlock) void z_stage1(const double2* __restrict__ p
   const int mcount = chunk > kBlock ? chunk / kBlock : 1;
   double tot = 0.0;
   double accm[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (tid < chunk) {
-    for (int m = 0; m < mcount; ++m) {
-      const double2 z = psi[base + tid + (uint64_t)m * kBlock];
-      const double p = fma(z.x, z.x, z.y * z.y);
-      tot += p;
+  for (int m0 = 0; m0 < mcount; m0 += kZPer) {
+    double2 z[kZPer];
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if ((m >> j) & 1) accm[j] += p;
+    for (int u = 0; u < kZPer; ++u) {
+      const int e = tid + (m0 + u) * kBlock;
+      z[u] = e < chunk ? psi[base + e] : make_double2(0.0, 0.0);
     }
+    double p[kZPer];
+#pragma unroll
+    for (int u = 0; u < kZPer; ++u) p[u] = fma(z[u].x, z[u].x, z[u].y * z[u].y);
+    const double s13 = p[1] + p[3], s57 = p[5] + p[7], s26 = p[2] + p[6];
+    const double odd = s13 + s57;
+    const double sum = ((p[0] + p[4]) + s26) + odd;
+    tot += sum;
+    accm[0] += odd;
+    accm[1] += s26 + (p[3] + p[7]);
+    accm[2] += (p[4] + p[6]) + s57;
+#pragma unroll
+    for (int j = 3; j < 8; ++j)
+      if ((m0 >> j) & 1) accm[j] += sum;
   }
   double v[17];
   v[0] = tot;
@@ -173,42 +221,37 @@ __global__ __launch_bounds__(kBlock) void z_stage1(const double2* __restrict__ p
   for (int j = 0; j < 8; ++j) v[9 + j] = accm[j];
   block_sum<17>(v, lds);
   if (tid == 0) {
-    double* out = partial + (uint64_t)blockIdx.x * (1 + kZChunkBits);
-    out[0] = v[0];
-    for (int b = 0; b < kZChunkBits; ++b) {
-      double s = 0.0;
-      if (b < 8 && b < c) s = v[1 + b];
-      else if (b >= 8 && b < c) s = v[9 + (b - 8)];
-      out[1 + b] = s;
-    }
+#pragma unroll
+    for (int b = 0; b <= kZChunkBits; ++b) partial[(uint64_t)b * gridDim.x + blockIdx.x] = v[b];
   }
 }
 
-// <Z> stage 2: out[a] = total - 2 S_{n-1-a}; high bits (>= c) come from the
-// block index.  One block; fixed summation order.
+// <Z> stage 2: block b writes out[n-1-b] = total - 2 S_b; high bits (>= c)
+// come from the block index.  Fixed summation order, the same total in every
+// block.  26 qubits: 5 us; one block walking the bits in turn took 37 us.
 __global__ __launch_bounds__(kBlock) void z_stage2(const double* __restrict__ partial, int nblk,
                                                   int n, int c, double* __restrict__ out) {
   __shared__ double lds[2 * 4];
-  __shared__ double s_tot;
+  const int b = blockIdx.x;
+  const double* sb = partial + (uint64_t)(1 + b) * nblk;
   double acc[2] = {0.0, 0.0};
-  for (int j = threadIdx.x; j < nblk; j += kBlock) acc[0] += partial[(uint64_t)j * (1 + kZChunkBits)];
-  block_sum<2>(acc, lds);
-  if (threadIdx.x == 0) s_tot = acc[0];
-  __syncthreads();
-  const double total = s_tot;
-  for (int b = 0; b < n; ++b) {
-    double s[2] = {0.0, 0.0};
-    for (int j = threadIdx.x; j < nblk; j += kBlock) {
-      const double* pj = partial + (uint64_t)j * (1 + kZChunkBits);
-      if (b < c)
-        s[0] += pj[1 + b];
-      else if (((uint64_t)j >> (b - c)) & 1)
-        s[0] += pj[0];
-    }
-    block_sum<2>(s, lds);
-    if (threadIdx.x == 0) out[n - 1 - b] = total - 2.0 * s[0];
-    __syncthreads();
+  for (int j = threadIdx.x; j < nblk; j += kBlock) {
+    const double t = partial[j];
+    acc[0] += t;
+    if (b < c) acc[1] += sb[j];
+    else if ((j >> (b - c)) & 1) acc[1] += t;
   }
+  block_sum<2>(acc, lds);
+  if (threadIdx.x == 0) out[n - 1 - b] = acc[0] - 2.0 * acc[1];
+}
+
+// Chunk bits of an n-qubit state: about 1024 chunks (four workgroups a CU)
+// of 2^11 (eight elements a lane) to 2^16 amplitudes.
+int z_chunk_bits(int n) {
+  int c = n - 10;
+  if (c < 11) c = 11;
+  if (c > kZChunkBits) c = kZChunkBits;
+  return c < n ? c : n;
 }
 
 template <int MODE>
@@ -290,7 +333,7 @@ int64_t qfx_reduce_workspace_bytes(int64_t len) {
   if (len > 1) {
     int n = 0;
     while (((int64_t)1 << n) < len) ++n;
-    const int c = n < kZChunkBits ? n : kZChunkBits;
+    const int c = z_chunk_bits(n);
     z = ((int64_t)1 << (n - c)) * (1 + kZChunkBits) * (int64_t)sizeof(double);
   }
   const int64_t r = (int64_t)kMaxRedBlocks * (int64_t)sizeof(double2);
@@ -300,6 +343,28 @@ int64_t qfx_reduce_workspace_bytes(int64_t len) {
 int qfx_inner(void* stream, void* result, const void* a, const void* b, int64_t len,
               void* workspace) {
   return run_reduce<0>(qfx::as_stream(stream), result, a, b, len, workspace, "qfx_inner");
+}
+
+int qfx_inner_permuted(void* stream, void* result, const void* a, const void* b, int n,
+                       const int* src_bit, void* workspace) {
+  const char* fn = "qfx_inner_permuted";
+  if (!result || !a || !b || !src_bit || !workspace)
+    return qfx::set_error(QFX_EINVAL, std::string(fn) + ": null pointer");
+  if (n < kPermT || n > QFX_MAX_QUBITS)
+    return qfx::set_error(QFX_ERANGE, std::string(fn) + ": n out of range");
+  int rc = qfx::check_permutation(n, src_bit, fn);
+  if (rc) return rc;
+  hipStream_t s = qfx::as_stream(stream);
+  const uint64_t ntiles = (uint64_t)1 << (n - kPermT);
+  const int nb = ntiles < (uint64_t)kMaxRedBlocks ? (int)ntiles : kMaxRedBlocks;
+  auto* part = static_cast<double2*>(workspace);
+  hipLaunchKernelGGL(inner_permuted_stage1, dim3(nb), dim3(kPermBlock), 0, s,
+                     static_cast<const double2*>(a), static_cast<const double2*>(b), ntiles, part,
+                     make_perm_tile(n, src_bit));
+  rc = qfx::check_launch(fn);
+  if (rc) return rc;
+  hipLaunchKernelGGL(reduce_stage2<0>, dim3(1), dim3(kBlock), 0, s, part, nb, result);
+  return qfx::check_launch(fn);
 }
 
 int qfx_expect_diag(void* stream, void* result, const void* psi, const void* diag, int64_t len,
@@ -350,14 +415,14 @@ int qfx_expect_z(void* stream, void* out, const void* psi, int n, void* workspac
   if (!out || !psi || !workspace) return qfx::set_error(QFX_EINVAL, "qfx_expect_z: null pointer");
   if (n < 1 || n > QFX_MAX_QUBITS) return qfx::set_error(QFX_ERANGE, "qfx_expect_z: n out of range");
   hipStream_t s = qfx::as_stream(stream);
-  const int c = n < kZChunkBits ? n : kZChunkBits;
+  const int c = z_chunk_bits(n);
   const uint64_t nblk = (uint64_t)1 << (n - c);
   auto* part = static_cast<double*>(workspace);
   hipLaunchKernelGGL(z_stage1, dim3((unsigned)nblk), dim3(kBlock), 0, s,
                      static_cast<const double2*>(psi), c, part);
   int rc = qfx::check_launch("qfx_expect_z");
   if (rc) return rc;
-  hipLaunchKernelGGL(z_stage2, dim3(1), dim3(kBlock), 0, s, part, (int)nblk, n, c,
+  hipLaunchKernelGGL(z_stage2, dim3(n), dim3(kBlock), 0, s, part, (int)nblk, n, c,
                      static_cast<double*>(out));
   return qfx::check_launch("qfx_expect_z");
 }

@@ -34,13 +34,19 @@ def permute_axes(tensor, perm):
         return tensor
     src = bk.as_device(tensor)
     out = src.new_empty(src.shape)
+    _native.call('qfx_permute_qubits', bk.stream_handle(),
+                 _native.ctypes.c_void_p(out.data_ptr()),
+                 _native.ctypes.c_void_p(src.data_ptr()), n, _native.int_array(_source_bits(perm)))
+    return out.view([2] * n)
+
+
+def _source_bits(perm):
+    """Index bit b of the new tensor is bit src[b] of the old one."""
+    n = len(perm)
     src_bit = [0] * n
     for a in range(n):
         src_bit[n - 1 - a] = n - 1 - perm[a]
-    _native.call('qfx_permute_qubits', bk.stream_handle(),
-                 _native.ctypes.c_void_p(out.data_ptr()),
-                 _native.ctypes.c_void_p(src.data_ptr()), n, _native.int_array(src_bit))
-    return out.view([2] * n)
+    return src_bit
 
 
 class QubitVector:
@@ -81,13 +87,17 @@ class QubitVector:
         qubits = tuple(qubits)
         if qubits == self.qubits:
             return self
+        return QubitVector(permute_axes(self.tensor, self._axes(qubits)), qubits)
+
+    def _axes(self, qubits: Qubits) -> List[int]:
+        """This tensor's axes in the label order ``qubits``."""
         N = self.qubit_nb
         assert len(qubits) == N
         indices = [self.qubits.index(q) for q in qubits]
         perm: List[int] = []
         for rr in range(self.rank):
             perm += [rr * N + idx for idx in indices]
-        return QubitVector(permute_axes(self.tensor, perm), qubits)
+        return perm
 
     @property
     def H(self) -> 'QubitVector':
@@ -113,8 +123,14 @@ def inner_product(vec0: QubitVector, vec1: QubitVector) -> bk.BKTensor:
     """Hilbert-Schmidt inner product (qubits.py:233-245)."""
     if vec0.rank != vec1.rank or vec0.qubit_nb != vec1.qubit_nb:
         raise ValueError('Incompatibly vectors. Qubits and rank must match')
-    vec1 = vec1.permute(vec0.qubits)
-    return bk.inner(vec0.tensor, vec1.tensor)
+    return _inner(vec0, vec1)
+
+
+def _inner(vec0: QubitVector, vec1: QubitVector) -> bk.BKTensor:
+    """sum conj(vec0) vec1 with vec1 in vec0's label order."""
+    if vec1.qubits == vec0.qubits:
+        return bk.inner(vec0.tensor, vec1.tensor)
+    return bk.inner_permuted(vec0.tensor, vec1.tensor, _source_bits(vec1._axes(vec0.qubits)))
 
 
 def outer_product(vec0: QubitVector, vec1: QubitVector) -> QubitVector:
@@ -137,9 +153,8 @@ def fubini_study_angle(vec0: QubitVector, vec1: QubitVector) -> bk.BKTensor:
     """Fubini-Study angle between vectors (qubits.py:282-307)."""
     if vec0.rank != vec1.rank or vec0.qubit_nb != vec1.qubit_nb:
         raise ValueError('Incompatibly vectors. Qubits and rank must match')
-    vec1 = vec1.permute(vec0.qubits)
     t0, t1 = vec0.tensor, vec1.tensor
-    hs01 = bk.inner(t0, t1)
+    hs01 = _inner(vec0, vec1)
     hs00 = bk.inner(t0, t0)
     hs11 = bk.inner(t1, t1)
     ratio = bk.absolute(hs01) / bk.sqrt(bk.absolute(hs00 * hs11))

@@ -173,6 +173,46 @@ def test_permute_qubits(bk):
     assert np.array_equal(got, np.transpose(a, perm))
 
 
+@pytest.mark.parametrize("n", [9, 10, 11, 13, 17])
+def test_permutations_by_tiles(bk, n):
+    # around the 10-bit tile: random orders, reversal, low and high halves
+    # exchanged, neighbours exchanged; the permuted inner product against both
+    from quantumflow_amd.qubits import QubitVector, inner_product, fubini_study_angle
+    rng = np.random.default_rng(60 + n)
+    a, b = rand_state(n, rng), rand_state(n, rng)
+    orders = [list(range(n))[::-1], list(range(n // 2, n)) + list(range(n // 2)),
+              [i ^ 1 if (i ^ 1) < n else i for i in range(n)]]
+    orders += [[int(i) for i in rng.permutation(n)] for _ in range(4)]
+    va = QubitVector(a, range(n))
+    for order in orders:
+        vb = QubitVector(b, order)
+        want = np.transpose(b, [order.index(q) for q in range(n)])
+        assert np.array_equal(bk.evaluate(vb.permute(range(n)).tensor), want), order
+        ip = np.vdot(a, want)
+        assert abs(complex(bk.evaluate(inner_product(va, vb))) - ip) <= 1e-14, order
+        ang = np.arccos(min(1.0, abs(ip) / np.sqrt(np.vdot(a, a).real * np.vdot(b, b).real)))
+        assert abs(float(bk.evaluate(fubini_study_angle(va, vb))) - ang) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [1, 3, 8, 10, 11, 12, 20, 21, 22])
+def test_reductions_at_chunk_edges(bk, n):
+    # 2^n around one block, one <Z> chunk of 2^11, and many
+    rng = np.random.default_rng(70 + n)
+    psi = rand_state(n, rng)
+    p = np.abs(psi) ** 2
+    d = rng.normal(size=[2] * n)
+    t = bk.astensorproduct(psi)
+    z = bk.evaluate(bk.expectation_z(t))
+    for a in range(n):
+        m = p.reshape(2 ** a, 2, -1).sum(axis=(0, 2))
+        # 2^n terms summed in a tree over at most 256 serial adds
+        assert abs(z[a] - (m[0] - m[1])) <= 1e-13, a
+    assert abs(float(bk.evaluate(bk.norm(t))) - p.sum()) <= 1e-13
+    assert abs(float(bk.evaluate(bk.expectation(d, t))) - (d * p).sum()) <= 1e-12
+    assert abs(complex(bk.evaluate(bk.inner(t, bk.astensorproduct(d.astype(complex)))))
+               - np.vdot(psi, d)) <= 1e-9
+
+
 def test_cut_table_bitwise(bk):
     import networkx as nx
     from quantumflow_amd.qaoa import graph_cuts
