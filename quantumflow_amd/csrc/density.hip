@@ -96,8 +96,12 @@ __global__ __launch_bounds__(kBlock) void axpy_kernel(double2* __restrict__ y,
 
 // out[r', c'] = sum_u rho[r, c], r = deposit(r', keep) | d(u), c =
 // deposit(c', keep) | d(u), d(u) = the u-th index over the traced bits
-// (stepped by one carry-add).  One thread per output element, terms in a
-// fixed order.
+// (stepped by one carry-add).  P = 2^lp lanes share an output element (terms
+// u = p, p + P, ..), which a fixed tree sums: with one lane an element, a
+// marginal of few qubits was a serial chain of 2^(n-m) dependent-latency loads
+// on a handful of lanes.  12 qubits down to 1: 248 us before, under 19 us (the
+// host's share of a call) now; to 11, where every lane has its own elements,
+// 33 us either way.
 __device__ __forceinline__ uint64_t deposit(uint64_t v, uint64_t mask) {
   uint64_t r = 0;
   for (uint64_t bit = 1; mask; bit <<= 1) {
@@ -110,22 +114,40 @@ __device__ __forceinline__ uint64_t deposit(uint64_t v, uint64_t mask) {
 
 __global__ __launch_bounds__(kBlock) void ptrace_kernel(double2* __restrict__ out,
                                                        const double2* __restrict__ rho, int n,
-                                                       uint32_t keep, int m) {
+                                                       uint32_t keep, int m, int lp) {
+  __shared__ double2 part[kBlock];
   const uint64_t dimk = (uint64_t)1 << m, dim = (uint64_t)1 << n, len = dimk * dimk;
   const uint64_t tr = (dim - 1) & ~(uint64_t)keep;
-  const uint64_t nt = (uint64_t)1 << (n - m);
-  for (uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x; t < len;
-       t += (uint64_t)gridDim.x * kBlock) {
-    const uint64_t r0 = deposit(t >> m, keep), c0 = deposit(t & (dimk - 1), keep);
+  const uint64_t nt = (uint64_t)1 << (n - m - lp);        // terms per lane
+  const unsigned per = kBlock >> lp;                      // elements per block
+  const unsigned p = threadIdx.x / per, j = threadIdx.x % per;
+  const uint64_t dp = deposit(p, tr);
+  uint64_t hi = tr;                                       // traced bits the lane steps
+  for (int b = 0; b < lp; ++b) hi &= hi - 1;
+  for (uint64_t t0 = (uint64_t)blockIdx.x * per; t0 < len; t0 += (uint64_t)gridDim.x * per) {
+    const uint64_t t = t0 + j;
     double re = 0.0, im = 0.0;
-    uint64_t d = 0;
-    for (uint64_t u = 0; u < nt; ++u) {
-      const double2 x = rho[(r0 | d) * dim + (c0 | d)];
-      re += x.x;
-      im += x.y;
-      d = ((d | ~tr) + 1) & tr;
+    if (t < len) {
+      const uint64_t r0 = deposit(t >> m, keep) | dp, c0 = deposit(t & (dimk - 1), keep) | dp;
+      uint64_t d = 0;
+#pragma unroll 4
+      for (uint64_t u = 0; u < nt; ++u) {
+        const double2 x = rho[(r0 | d) * dim + (c0 | d)];
+        re += x.x;
+        im += x.y;
+        d = ((d | ~hi) + 1) & hi;
+      }
     }
-    out[t] = double2{re, im};
+    part[threadIdx.x] = double2{re, im};
+    for (unsigned h = kBlock / 2; h >= per; h >>= 1) {
+      __syncthreads();
+      if (threadIdx.x < h) {
+        part[threadIdx.x].x += part[threadIdx.x + h].x;
+        part[threadIdx.x].y += part[threadIdx.x + h].y;
+      }
+    }
+    if (p == 0 && t < len) out[t] = part[j];
+    __syncthreads();
   }
 }
 
@@ -191,9 +213,15 @@ int qfx_density_partial_trace(void* stream, void* out, const void* rho, int n,
   if (keep_mask == 0 || (keep_mask >> n) != 0)
     return qfx::set_error(QFX_EINVAL, "qfx_density_partial_trace: bad keep mask");
   const int m = __builtin_popcount(keep_mask);
-  hipLaunchKernelGGL(ptrace_kernel, dim3(grid_for((uint64_t)1 << (2 * m))), dim3(kBlock), 0,
+  // lanes per element: until 2^17 lanes (two waves a SIMD) or every term has
+  // one, 256 at most
+  int lp = 17 - 2 * m;
+  if (lp > n - m) lp = n - m;
+  if (lp > 8) lp = 8;
+  if (lp < 0) lp = 0;
+  hipLaunchKernelGGL(ptrace_kernel, dim3(grid_for((uint64_t)1 << (2 * m + lp))), dim3(kBlock), 0,
                      qfx::as_stream(stream), static_cast<double2*>(out),
-                     static_cast<const double2*>(rho), n, keep_mask, m);
+                     static_cast<const double2*>(rho), n, keep_mask, m, lp);
   return qfx::check_launch("ptrace_kernel");
 }
 

@@ -169,6 +169,21 @@ def test_partial_trace_matches_oracle(qf, traced):
         rho.partial_trace(list('abcdef'))
 
 
+@pytest.mark.parametrize("n,kept", [(1, [0]), (2, [1]), (8, [0]), (8, [7]), (9, [3]), (10, [0, 9]),
+                                    (8, [0, 2, 4, 6]), (9, [1, 2, 3, 4, 5, 6, 7, 8])])
+def test_partial_trace_split_terms(qf, n, kept):
+    # 1 to 256 lanes share an element; every split and both ends of the bits
+    rng = np.random.default_rng(90 + n + len(kept))
+    m0 = _rand_density(n, rng)
+    rho = qf.Density(m0.reshape([2] * (2 * n)))
+    gone = [q for q in range(n) if q not in kept]
+    out = rho.partial_trace(gone) if gone else rho
+    ref = m0.reshape([2] * (2 * n))
+    for q in reversed(gone):
+        ref = np.trace(ref, axis1=q, axis2=ref.ndim // 2 + q)
+    assert np.max(np.abs(_mat(out) - ref.reshape(2 ** len(kept), -1))) <= 1e-14
+
+
 def test_channel_evolve_and_composition(qf):
     """Channel.evolve runs the superoperator as one gate on the row and
     column axes (dense 2-qubit, monomial 4-qubit and, for a 2-qubit Kraus
