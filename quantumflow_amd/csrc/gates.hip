@@ -18,6 +18,7 @@
 namespace {
 
 constexpr int kBlock = 256;
+constexpr int kCus = 256;
 
 template <int K>
 struct DenseArg {
@@ -125,8 +126,8 @@ __global__ __launch_bounds__(kBlock) void sparse_kernel(double2* out, const doub
   }
 }
 
-// General dense gate with the matrix in device memory; one output amplitude
-// per lane.  Needs out != in.  The 2^k column offsets are built in LDS.
+// Dense gate of up to 3 qubits with the matrix in device memory; one output
+// amplitude per lane.  Needs out != in.  The 2^k column offsets are built in LDS.
 struct DevTargets {
   int t[QFX_MAX_DENSE_K];  // bit of gate qubit j (MSB first)
 };
@@ -155,6 +156,166 @@ __global__ __launch_bounds__(kBlock) void dense_dev_kernel(double2* __restrict__
   const double2* row = m + (uint64_t)r * D;
   for (int c = 0; c < D; ++c) cmac(acc, row[c], in[base + s_off[c]]);
   out[i] = acc;
+}
+
+// Dense gates of 4 to 12 qubits on the matrix cores: Y = M X with X the
+// 2^k x 2^(n-k) matrix of the state's amplitude groups, in complex products of
+// four v_mfma_f64_16x16x4f64 each (operand layout: lane l holds A[l%16][l/16],
+// B[l/16][l%16] and, in register j, D[4j + l/16][l%16]).
+//
+// A workgroup computes R gate rows of C groups (R = 2^k up to 64, so gates of
+// up to 6 qubits read the state once) and walks the gate's columns 16 at a
+// time; the chunk of X and M for the next step is in flight while the current
+// one is multiplied out of LDS.  Both matrices are indexed with the targets in
+// ascending order, so that a chunk holds the four lowest targets together
+// with the C lowest groups: its loads run over contiguous memory whichever
+// bits those are (M's rows and columns are permuted to match).  Arithmetic is
+// 8 2^k flops an amplitude: memory bounds gates of 4 and 5 qubits, the matrix
+// cores those from 7 on.  8 qubits of 20: 54 us, 39 TFLOP/s (one output
+// amplitude a lane: 250 us on high bits, 564 us on low ones); 10 of 24 qubits
+// 2.3 ms, 60 TFLOP/s (21.3 ms); 4 of 24 qubits 107-133 us, 4.0-5.0 TB/s
+// (383-653 us).
+struct GemmArg {
+  int k;
+  int epos[11];               // chunk element bit t -> state index bit
+  int eslot[11];              //                     -> bit of (c << log2 C | g)
+  unsigned einvalid;          // element bits past the state's groups
+  int gbits;                  // group bits inside a tile (log2 C unless n-k is less)
+  int gpos[7];                // their index bits
+  int sorted[QFX_MAX_DENSE_K];   // targets ascending
+  int mbit[QFX_MAX_DENSE_K];     // bit j of the ascending order -> matrix index bit
+  int nrest;
+  int rest[QFX_MAX_QUBITS];   // index bits of the tile number
+};
+
+typedef double v4d __attribute__((ext_vector_type(4)));
+constexpr int kKc = 16;       // gate columns per step
+
+template <int R, int C>
+__global__ __launch_bounds__(kBlock) void dense_mfma_kernel(double2* __restrict__ out,
+                                                           const double2* __restrict__ in,
+                                                           unsigned ntiles, GemmArg a,
+                                                           const double2* __restrict__ m) {
+  constexpr int kLc = C == 128 ? 7 : 6;
+  constexpr int NX = kKc * C / kBlock, NM = kKc * R / kBlock;
+  constexpr int WR = R < 32 ? R : 32, kRowWaves = R / WR;
+  constexpr int WC = C * kRowWaves / 4;               // one wave: WR x WC
+  constexpr int RB = WR / 16, CB = WC / 16;
+  __shared__ v2d xs[kKc * C], ms[kKc * R];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int q = lane >> 4, col = lane & 15;
+  const int D = 1 << a.k, nrt = D / R;
+  // tiles that share their groups follow each other on one XCD (blocks are
+  // dealt to the 8 XCDs in turn)
+  unsigned ct, rt;
+  if ((ntiles & 7u) == 0) {
+    ct = (blockIdx.x / (8u * nrt)) * 8u + (blockIdx.x & 7u);
+    rt = (blockIdx.x >> 3) % nrt;
+  } else {
+    ct = blockIdx.x / nrt;
+    rt = blockIdx.x % nrt;
+  }
+  uint64_t base = 0;
+  for (int b = 0; b < a.nrest; ++b) base |= (uint64_t)((ct >> b) & 1u) << a.rest[b];
+  // this lane's chunk elements tid + 256 u: state offsets and LDS slots
+  uint64_t xoff[NX];
+  int xslot[NX];
+  bool xin[NX];
+#pragma unroll
+  for (int u = 0; u < NX; ++u) {
+    const unsigned e = tid + kBlock * u;
+    uint64_t o = 0;
+    unsigned sl = 0;
+#pragma unroll
+    for (int t = 0; t < 4 + kLc; ++t) {
+      const unsigned bit = (e >> t) & 1u;
+      o |= (uint64_t)bit << a.epos[t];
+      sl |= bit << a.eslot[t];
+    }
+    xin[u] = (e & a.einvalid) == 0;
+    xoff[u] = xin[u] ? o : 0;
+    const unsigned c = sl >> kLc, g = sl & (C - 1);
+    xslot[u] = (int)(c * C + (g ^ c));   // lanes differing in c on different banks
+  }
+  auto mat_index = [&](unsigned v, int lo) {
+    unsigned r = 0;
+    for (int j = lo; j < a.k; ++j) r |= ((v >> j) & 1u) << a.mbit[j];
+    return r;
+  };
+  uint64_t moff[NM];
+  int mslot[NM];
+#pragma unroll
+  for (int u = 0; u < NM; ++u) {
+    const unsigned c = tid & 15u, r = (tid >> 4) + 16u * u;
+    moff[u] = (uint64_t)mat_index(rt * R + r, 0) * D + mat_index(c, 0);
+    mslot[u] = (int)(c * R + (r ^ c));
+  }
+  v2d x[NX], mm[NM];
+  auto fetch = [&](unsigned chunk) {
+    uint64_t co = 0;
+    for (int j = 4; j < a.k; ++j) co |= (uint64_t)((chunk >> (j - 4)) & 1u) << a.sorted[j];
+    const v2d* p = reinterpret_cast<const v2d*>(in) + base + co;
+    const v2d* pm = reinterpret_cast<const v2d*>(m) + mat_index(chunk << 4, 4);
+#pragma unroll
+    for (int u = 0; u < NX; ++u) x[u] = xin[u] ? p[xoff[u]] : v2d{0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < NM; ++u) mm[u] = pm[moff[u]];
+  };
+  const int wr = (wave % kRowWaves) * WR, wc = (wave / kRowWaves) * WC;
+  v4d re[RB][CB], im[RB][CB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j) re[i][j] = im[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  const unsigned nchunk = (unsigned)D / kKc;
+  fetch(0);
+  for (unsigned ch = 0; ch < nchunk; ++ch) {
+#pragma unroll
+    for (int u = 0; u < NX; ++u) xs[xslot[u]] = x[u];
+#pragma unroll
+    for (int u = 0; u < NM; ++u) ms[mslot[u]] = mm[u];
+    __syncthreads();
+    if (ch + 1 < nchunk) fetch(ch + 1);
+#pragma unroll
+    for (int ks = 0; ks < kKc / 4; ++ks) {
+      const int c = 4 * ks + q;
+      v2d av[RB], bv[CB];
+#pragma unroll
+      for (int i = 0; i < RB; ++i) av[i] = ms[c * R + ((wr + 16 * i + col) ^ c)];
+#pragma unroll
+      for (int j = 0; j < CB; ++j) bv[j] = xs[c * C + ((wc + 16 * j + col) ^ c)];
+#pragma unroll
+      for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+          re[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].x, bv[j].x, re[i][j], 0, 0, 0);
+          im[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].x, bv[j].y, im[i][j], 0, 0, 0);
+          re[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-av[i].y, bv[j].y, re[i][j], 0, 0, 0);
+          im[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].y, bv[j].x, im[i][j], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+  }
+  // row wr + 16 i + 4 j + q, group wc + 16 cb + col
+  const uint64_t qoff = ((uint64_t)(q & 1) << a.sorted[0]) | ((uint64_t)(q >> 1) << a.sorted[1]);
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) {
+    const unsigned g = wc + 16 * cb + col;
+    if (g >> a.gbits) continue;
+    uint64_t go = base | qoff;
+    for (int t = 0; t < a.gbits; ++t) go |= (uint64_t)((g >> t) & 1u) << a.gpos[t];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      const unsigned r = rt * R + wr + 16 * i;
+      uint64_t ro = 0;
+      for (int t = 4; t < a.k; ++t) ro |= (uint64_t)((r >> t) & 1u) << a.sorted[t];
+      v2d* p = reinterpret_cast<v2d*>(out) + (go | ro);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        p[((uint64_t)(j & 1) << a.sorted[2]) | ((uint64_t)(j >> 1) << a.sorted[3])] =
+            v2d{re[i][cb][j], im[i][cb][j]};
+    }
+  }
 }
 
 // out[i] = in[j] where bit src[b] of j equals bit b of i (a relabelling of
@@ -252,6 +413,60 @@ int launch_sparse(hipStream_t s, double2* out, const double2* in, int n, int k,
   return qfx::set_error(QFX_ERANGE, "sparse gate width out of range");
 }
 
+template <int R, int C>
+int launch_mfma(hipStream_t s, double2* out, const double2* in, int n, int k, const int* targets,
+                const double2* m) {
+  constexpr int kLc = C == 128 ? 7 : 6;
+  GemmArg a;
+  std::memset(&a, 0, sizeof(a));
+  a.k = k;
+  qfx::sort_bits(k, targets, a.sorted);
+  for (int j = 0; j < k; ++j)
+    for (int t = 0; t < k; ++t)
+      if (targets[t] == a.sorted[j]) a.mbit[j] = k - 1 - t;   // gate qubit 0 is the MSB
+  uint64_t tmask = 0;
+  for (int j = 0; j < k; ++j) tmask |= (uint64_t)1 << targets[j];
+  for (int b = 0; b < n; ++b) {
+    if ((tmask >> b) & 1) continue;
+    if (a.gbits < kLc) a.gpos[a.gbits++] = b;
+    else a.rest[a.nrest++] = b;
+  }
+  // chunk elements in address order: columns 0..3 of the gate and the groups
+  int t = 0;
+  for (int b = 0; b < n; ++b) {
+    for (int j = 0; j < 4; ++j)
+      if (a.sorted[j] == b) { a.epos[t] = b; a.eslot[t++] = kLc + j; }
+    for (int j = 0; j < a.gbits; ++j)
+      if (a.gpos[j] == b) { a.epos[t] = b; a.eslot[t++] = j; }
+  }
+  for (int j = a.gbits; j < kLc; ++j) {      // groups that the state does not have
+    a.einvalid |= 1u << t;
+    a.epos[t] = 0;
+    a.eslot[t++] = j;
+  }
+  const unsigned ntiles = 1u << a.nrest;
+  const unsigned blocks = ntiles * (unsigned)((1 << k) / R);
+  hipLaunchKernelGGL((dense_mfma_kernel<R, C>), dim3(blocks), dim3(kBlock), 0, s, out, in, ntiles,
+                     a, m);
+  return qfx::check_launch("dense_mfma_kernel");
+}
+
+// The largest tile whose grid still covers the 256 CUs, else 16 x 64, whose
+// step is a quarter as long and whose grid is larger (8 qubits of 16: 47 us
+// with 16 workgroups of 64 x 64, 22 us with 64 of 16 x 64; 10 of 18: 179 and
+// 87 us, 64 and 256 workgroups).
+int launch_wide(hipStream_t s, double2* out, const double2* in, int n, int k, const int* targets,
+                const double2* m) {
+  const int gb = n - k;
+  auto blocks = [&](int row_bits, int col_bits) {
+    return (int64_t)1 << ((k > row_bits ? k - row_bits : 0) + (gb > col_bits ? gb - col_bits : 0));
+  };
+  if (k >= 6 && blocks(6, 6) >= kCus) return launch_mfma<64, 64>(s, out, in, n, k, targets, m);
+  if (k == 5 && blocks(5, 7) >= kCus) return launch_mfma<32, 128>(s, out, in, n, k, targets, m);
+  if (k == 4 && blocks(4, 7) >= kCus) return launch_mfma<16, 128>(s, out, in, n, k, targets, m);
+  return launch_mfma<16, 64>(s, out, in, n, k, targets, m);
+}
+
 bool is_one(const qfx_c128& z) { return z.re == 1.0 && z.im == 0.0; }
 
 // Build SparseArg for a diagonal (src == NULL) or monomial gate.
@@ -307,6 +522,10 @@ int qfx_apply_matrix_dev(void* stream, void* out, const void* in, int n, int k,
   if (!out || !in || !matrix)
     return qfx::set_error(QFX_EINVAL, "qfx_apply_matrix_dev: null pointer");
   if (out == in) return qfx::set_error(QFX_EINVAL, "qfx_apply_matrix_dev: out must not alias in");
+  if (k >= 4)
+    return launch_wide(qfx::as_stream(stream), static_cast<double2*>(out),
+                       static_cast<const double2*>(in), n, k, targets,
+                       static_cast<const double2*>(matrix));
   DevTargets tg;
   std::memset(&tg, 0, sizeof(tg));
   for (int j = 0; j < k; ++j) tg.t[j] = targets[j];

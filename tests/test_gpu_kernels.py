@@ -67,6 +67,30 @@ def test_dense_device_matrix(bk, k):
     assert np.max(np.abs(got - ref)) <= TOL
 
 
+@pytest.mark.parametrize("k", [4, 5, 6, 7, 8])
+@pytest.mark.parametrize("extra", [0, 1, 2, 3, 5, 6, 7, 8, 10])
+def test_wide_dense_gates(bk, k, extra):
+    # matrix-core and plain kernel on either side of the group tile (2^6 or
+    # 2^7), targets lowest, highest, spread and in any order
+    import torch
+    n = k + extra
+    if n > 16:
+        pytest.skip("covered by smaller k")
+    rng = np.random.default_rng(1000 * k + extra)
+    psi = rand_state(n, rng)
+    u = rand_unitary(k, rng)
+    for axes in (list(range(k)), list(range(n))[::-1][:k], [int(a) for a in rng.permutation(n)[:k]],
+                 sorted(int(a) for a in rng.permutation(n)[:k])):
+        rest = [a for a in range(n) if a not in axes]
+        x = np.transpose(psi, axes + rest).reshape(2 ** k, -1)
+        want = np.transpose((u @ x).reshape([2] * n), np.argsort(axes + rest))
+        got = bk.evaluate(bk.tensormul(torch.from_numpy(u.reshape([2] * (2 * k))).cuda(),
+                                       bk.astensorproduct(psi), axes))
+        # a unit row times a part of a unit vector: 4 2^k roundings of 2^-53,
+        # on either side
+        assert np.max(np.abs(got - want)) <= 8 * 2 ** k * 2.0 ** -53, axes
+
+
 @pytest.mark.parametrize("name,params,k", [
     ('RZ', (0.731,), 1), ('PHASE', (2.1,), 1), ('CZ', (), 2), ('ZZ', (0.37,), 2),
     ('CPHASE', (1.3,), 2), ('S', (), 1), ('T', (), 1)])
