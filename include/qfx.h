@@ -94,6 +94,24 @@ int qfx_apply_monomial_inplace(void* stream, void* state, int n, int k,
                                const int* targets, const int* src,
                                const qfx_c128* phase);
 
+/* ---- runs of gates (Circuit.run / evolve / asgate,
+ *      quantumflow/circuits.py:87-127) ------------------------------------ */
+#define QFX_GATE_DENSE 0    /* coef: row-major 2^k x 2^k matrix, k <= 3      */
+#define QFX_GATE_DIAGONAL 1 /* coef: 2^k diagonal entries, k <= 4            */
+#define QFX_GATE_MONOMIAL 2 /* src: source row of each row, coef: phases of  */
+                            /* the rows or NULL, k <= 4                      */
+typedef struct {
+  int32_t kind, k;
+  const qfx_c128* coef; /* host */
+  const int32_t* src;   /* host */
+} qfx_gate;
+
+/* out = the gates applied to in, in order (gates that share no bit may change
+ * places).  gates: host array of ngates >= 1 host records; bits: host, the
+ * targets of all gates one after another.  out == in is allowed. */
+int qfx_apply_gates(void* stream, void* out, const void* in, int n, int ngates,
+                    const qfx_gate* const* gates, const int* bits);
+
 /* ---- readouts (quantumflow/states.py:113-147, numpybk.py:125-128,
  *      quantumflow/qubits.py:180-182) ------------------------------------- */
 

@@ -34,6 +34,11 @@ class QfxTileOp(ctypes.Structure):
                 ('lds', ctypes.c_uint32 * 10)]
 
 
+class QfxGate(ctypes.Structure):
+    _fields_ = [('kind', ctypes.c_int32), ('k', ctypes.c_int32), ('coef', ctypes.c_void_p),
+                ('src', ctypes.c_void_p)]
+
+
 _vp = ctypes.c_void_p
 _i = ctypes.c_int
 _i64 = ctypes.c_int64
@@ -53,6 +58,7 @@ SIGNATURES = {
     'qfx_apply_monomial': (_i, [_vp, _vp, _vp, _i, _i, _ip, _ip, _cp]),
     'qfx_apply_diagonal_inplace': (_i, [_vp, _vp, _i, _i, _ip, _cp]),
     'qfx_apply_monomial_inplace': (_i, [_vp, _vp, _i, _i, _ip, _ip, _cp]),
+    'qfx_apply_gates': (_i, [_vp, _vp, _vp, _i, _i, ctypes.POINTER(_vp), _ip]),
     'qfx_reduce_workspace_bytes': (_i64, [_i64]),
     'qfx_inner': (_i, [_vp, _vp, _vp, _vp, _i64, _vp]),
     'qfx_inner_permuted': (_i, [_vp, _vp, _vp, _vp, _i, _ip, _vp]),

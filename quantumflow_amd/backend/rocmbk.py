@@ -337,7 +337,7 @@ class GateKind:
     """Classification of a 2^k x 2^k gate matrix for kernel selection."""
     DENSE, DIAGONAL, MONOMIAL = 'dense', 'diagonal', 'monomial'
 
-    __slots__ = ('kind', 'k', 'matrix', 'diag', 'src', 'phase')
+    __slots__ = ('kind', 'k', 'matrix', 'diag', 'src', 'phase', '_record')
 
     def __init__(self, matrix):
         m = np.asarray(matrix, dtype=_NP_CTYPE)
@@ -345,18 +345,40 @@ class GateKind:
         m = m.reshape(dim, dim)
         self.k = int(math.log2(dim))
         self.matrix = np.ascontiguousarray(m)
-        self.diag = self.src = self.phase = None
-        nz = m != 0
-        if self.k <= 5 and not np.any(nz & ~np.eye(dim, dtype=bool)):
+        self.diag = self.src = self.phase = self._record = None
+        self.kind = GateKind.DENSE
+        if self.k > 5:
+            return
+        # the columns of each row's nonzero entries: matrices of this size are
+        # read faster as lists than by numpy calls
+        rows = [[c for c, z in enumerate(row) if z != 0] for row in m.tolist()]
+        if all(cols == [r] or not cols for r, cols in enumerate(rows)):
             self.kind = GateKind.DIAGONAL
-            self.diag = np.diag(m).copy()
-        elif self.k <= 5 and np.all(nz.sum(axis=1) == 1) and np.all(nz.sum(axis=0) == 1):
+            self.diag = m.diagonal().copy()
+        elif all(len(cols) == 1 for cols in rows) and \
+                len({cols[0] for cols in rows}) == dim:
             self.kind = GateKind.MONOMIAL
-            self.src = np.argmax(nz, axis=1).astype(np.int32)
+            self.src = np.array([cols[0] for cols in rows], dtype=np.int32)
             ph = m[np.arange(dim), self.src]
-            self.phase = None if np.all(ph == 1.0) else ph
-        else:
-            self.kind = GateKind.DENSE
+            self.phase = None if all(z == 1.0 for z in ph.tolist()) else ph
+
+    @property
+    def listable(self):
+        """Whether qfx_apply_gates takes this gate."""
+        return self.k <= (3 if self.kind == GateKind.DENSE else 4)
+
+    def record(self):
+        """(host address of the gate's qfx_gate record, the record and the
+        arrays that it points to)."""
+        if self._record is None:
+            code, coef = {GateKind.DENSE: (0, self.matrix), GateKind.DIAGONAL: (1, self.diag),
+                          GateKind.MONOMIAL: (2, self.phase)}[self.kind]
+            coef = None if coef is None else np.ascontiguousarray(coef)
+            src = None if self.src is None else np.ascontiguousarray(self.src, dtype=np.int32)
+            rec = _native.QfxGate(code, self.k, None if coef is None else coef.ctypes.data,
+                                  None if src is None else src.ctypes.data)
+            self._record = (_native.ctypes.addressof(rec), rec, coef, src)
+        return self._record
 
 
 def classify(matrix):
@@ -394,6 +416,22 @@ def apply_gate(out, state, n, bits, kind, inplace_sparse=False):
         else:
             _native.call('qfx_apply_matrix_dev', s, _ptr(out), _ptr(state), n, k, tb, _ptr(dm))
     return out
+
+
+def apply_gates(tensor: BKTensor, kinds: typing.List[GateKind],
+                bits: typing.List[int]) -> BKTensor:
+    """The gates of ``kinds`` (each listable) applied to a [2]*N tensor in
+    order, many a launch (qfx_apply_gates); ``bits`` holds their index bits
+    (N-1-axis) one gate after another.  Returns a new [2]*N device tensor."""
+    state = as_device(tensor)
+    n = rank(tensor)
+    out = torch.empty_like(state)
+    recs = [k.record() for k in kinds]          # keeps the arrays alive over the call
+    m = len(recs)
+    _native.call('qfx_apply_gates', stream_handle(), _ptr(out), _ptr(state), n, m,
+                 (_native.ctypes.c_void_p * m)(*[r[0] for r in recs]),
+                 (_native.ctypes.c_int * len(bits))(*bits))
+    return out.view([2] * n)
 
 
 def tensormul(tensor0: BKTensor, tensor1: BKTensor,
@@ -601,6 +639,14 @@ def sample_expectation(diag_hermitian: BKTensor, tensor: BKTensor, trials: int,
     d = _real_diag(diag_hermitian, a.numel())
     idx = sample_indices(a, trials, seed)
     return torch.sum(d[idx]) / int(trials)
+
+
+def identity_tensor(n: int) -> BKTensor:
+    """The identity on n qubits as a [2]*2n tensor, filled on the device."""
+    _ensure_device()
+    t = torch.empty(4 ** n, dtype=CTYPE, device=DEVICE)
+    _native.call('qfx_density_identity', stream_handle(), _ptr(t), n, 1.0)
+    return t.view([2] * (2 * n))
 
 
 def zero_state_tensor(n: int) -> BKTensor:

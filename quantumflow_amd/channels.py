@@ -149,13 +149,19 @@ def state_asdensity(ket: State) -> Density:
     return Density(rho.view([2] * (2 * n)), ket.qubits, ket._memory)
 
 
+def _kron_conj(m):
+    """m (x) conj(m)."""
+    d = m.shape[0]
+    return (m[:, None, :, None] * np.conj(m)[None, :, None, :]).reshape(d * d, d * d)
+
+
 def _one_pass_kind(m):
     """The kernel class of U (x) conj(U) if one gate kernel takes it, else
     None."""
     k = int(round(np.log2(m.shape[0])))
     if 2 * k > 5:
         return None
-    kind = bk.classify(np.kron(m, np.conj(m)))
+    kind = bk.classify(_kron_conj(m))
     return kind if 2 * k <= 3 or kind.kind != kind.DENSE else None
 
 
@@ -182,6 +188,30 @@ def gate_evolve(gate: Gate, rho: Density) -> Density:
     t = bk.tensormul(m.reshape([2] * (2 * k)), rho.tensor, idx)
     t = bk.tensormul(np.conj(m).reshape([2] * (2 * k)), t, cols)
     return Density(t, rho.qubits, rho._memory)
+
+
+def evolve_kinds(elem):
+    """How the gate-list kernel evolves a density by ``elem``: [(kernel class,
+    axes)] with axes 'rows', 'cols' or 'both' (rows then columns) of the
+    element's qubits, the gates that gate_evolve, Kraus.evolve and
+    Channel.evolve apply one pass each; None where it does not take them or
+    the element's evolve is its own."""
+    method = getattr(type(elem), 'evolve', None)
+    if isinstance(elem, Gate) and method is Gate.evolve:
+        if elem.qubit_nb > 3:
+            return None
+        m = elem.matrix
+        kind = _one_pass_kind(m)
+        if kind is not None:
+            return [(kind, 'both')]
+        return [(elem.kind, 'rows'), (bk.classify(np.conj(m)), 'cols')]
+    if isinstance(elem, Kraus) and method is Kraus.evolve:
+        kind = elem._one_pass_kind()
+        return None if kind is None else [(kind, 'both')]
+    if isinstance(elem, Channel) and method is Channel.evolve:
+        kind = bk.classify(elem._mat)
+        return [(kind, 'both')] if kind.listable else None
+    return None
 
 
 class Channel(Operation):
@@ -368,9 +398,19 @@ class Kraus(Operation):
         K = len(qubits)
         S = np.zeros((4 ** K, 4 ** K), dtype=np.complex128)
         for op, w in zip(self.operators, self.weights):
-            m = _embed(op.matrix, [qubits.index(q) for q in op.qubits], K)
-            S += w * np.kron(m, np.conj(m))
+            m = op.matrix if op.qubits == qubits else \
+                _embed(op.matrix, [qubits.index(q) for q in op.qubits], K)
+            S += w * _kron_conj(m)
         return S
+
+    def _one_pass_kind(self):
+        """The kernel class of the channel's superoperator if one gate kernel
+        takes it, else None."""
+        K = len(self.qubits)
+        if 2 * K > 5:
+            return None
+        kind = bk.classify(self.superoperator())
+        return kind if 2 * K <= 3 or kind.kind != kind.DENSE else None
 
     def evolve(self, rho: Density) -> Density:
         """Weighted sum of the operators' evolutions (channels.py:74-80).
@@ -378,14 +418,12 @@ class Kraus(Operation):
         channels: a dense 2-qubit gate on the row and column axes), that is
         one pass over the density; otherwise each operator's evolution is
         accumulated by weighted sums."""
-        qubits = self.qubits
-        if 2 * len(qubits) <= 5:
-            kind = bk.classify(self.superoperator())
-            if 2 * len(qubits) <= 3 or kind.kind != kind.DENSE:
-                N = rho.qubit_nb
-                idx = [rho.qubits.index(q) for q in qubits]
-                t = bk.tensormul(kind, rho.tensor, idx + [N + i for i in idx])
-                return Density(t, rho.qubits, rho._memory)
+        kind = self._one_pass_kind()
+        if kind is not None:
+            N = rho.qubit_nb
+            idx = [rho.qubits.index(q) for q in self.qubits]
+            t = bk.tensormul(kind, rho.tensor, idx + [N + i for i in idx])
+            return Density(t, rho.qubits, rho._memory)
         out = torch.zeros(4 ** rho.qubit_nb, dtype=torch.complex128, device=bk.DEVICE)
         for op, w in zip(self.operators, self.weights):
             term = bk.as_device(op.evolve(rho).tensor)

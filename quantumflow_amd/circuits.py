@@ -4,6 +4,7 @@
 For plain Gates on a state of at least ``FUSED_MIN_QUBITS`` qubits it hands
 the whole gate list to the fused executor (quantumflow_amd.executor), which
 plans LDS-tiled passes and fused dense blocks and runs them on the GPU;
+on smaller states, runs of gates go to the gate-list kernel, many a launch;
 ``run(ket, fused=False)`` forces the plain path, one kernel per gate.
 """
 
@@ -12,6 +13,7 @@ from itertools import chain
 from math import pi
 from typing import Dict, Iterable, Iterator, Sequence, Type
 
+from . import backend as bk
 from . import config
 from .gates import control_gate, identity_gate
 from .ops import Gate, Operation
@@ -24,6 +26,49 @@ __all__ = ['Circuit', 'count_operations', 'map_gate', 'qft_circuit',
            'phase_estimation_circuit', 'addition_circuit', 'ghz_circuit']
 
 FUSED_MIN_QUBITS = 14
+
+
+def _listed(elem, method):
+    """The gate's kernel class if ``elem`` is a Gate whose ``method`` is
+    Gate's own and the gate-list kernel takes it, else None."""
+    if not isinstance(elem, Gate) or getattr(type(elem), method) is not getattr(Gate, method):
+        return None
+    if elem._host is None and elem.qubit_nb > 3:
+        return None                             # stays on the device
+    kind = elem.kind
+    return kind if kind.listable else None
+
+
+def _runs(elements, item):
+    """Split ``elements`` into maximal runs: yields (list of (elem, item(elem))
+    pairs, None) for runs of at least two elements with an item, else
+    (None, elem)."""
+    run = []
+    for elem in chain(elements, [None]):
+        it = item(elem) if elem is not None else None
+        if it is not None:
+            run.append((elem, it))
+            continue
+        if len(run) > 1:
+            yield run, None
+        elif run:
+            yield None, run[0][0]
+        run = []
+        if elem is not None:
+            yield None, elem
+
+
+def _bits_of(qubits):
+    """Index bit of each qubit label of a state."""
+    n = len(qubits)
+    return {q: n - 1 - i for i, q in enumerate(qubits)}
+
+
+def _lookup(bit_of, qubits):
+    try:
+        return [bit_of[q] for q in qubits]
+    except KeyError as e:
+        raise ValueError('qubit %r is not in the state' % (e.args[0],)) from None
 
 
 class Circuit(Operation):
@@ -85,8 +130,24 @@ class Circuit(Operation):
         default |0...0><0...0| on the circuit's qubits."""
         if rho is None:
             rho = zero_state(qubits=self.qubits).asdensity()
-        for elem in self.elements:
-            rho = elem.evolve(rho)
+        from .channels import evolve_kinds, Density
+        for run, elem in _runs(self.elements, evolve_kinds):
+            if run is None:
+                rho = elem.evolve(rho)
+                continue
+            # each element's kernel gates act on its qubits' row axes, then
+            # (or also) on their column axes
+            n = rho.qubit_nb
+            bit_of = _bits_of(rho.qubits)
+            kinds, bits = [], []
+            for e, gates in run:
+                cols = _lookup(bit_of, e.qubits)
+                rows = [b + n for b in cols]
+                for kind, where in gates:
+                    kinds.append(kind)
+                    bits += rows + cols if where == 'both' else \
+                        (rows if where == 'rows' else cols)
+            rho = Density(bk.apply_gates(rho.tensor, kinds, bits), rho.qubits, rho._memory)
         return rho
 
     def run(self, ket: State = None, fused: bool = None) -> State:
@@ -99,6 +160,8 @@ class Circuit(Operation):
         if ket is None:
             ket = zero_state(qubits=self.qubits)
         if fused is None:
+            if config.FUSION and 0 < ket.qubit_nb < FUSED_MIN_QUBITS:
+                return self._run_small(ket)
             fused = config.FUSION and ket.qubit_nb >= FUSED_MIN_QUBITS
         if not fused:
             for elem in self.elements:
@@ -119,12 +182,44 @@ class Circuit(Operation):
                 ket = elem.run(ket)
         return ket
 
+    def _run_small(self, ket: State) -> State:
+        """Runs of gates through the gate-list kernel, other elements one by
+        one in order."""
+        def flat(circ):
+            for elem in circ.elements:
+                if isinstance(elem, Circuit) and type(elem).run is Circuit.run:
+                    yield from flat(elem)
+                else:
+                    yield elem
+        for run, elem in _runs(flat(self), lambda e: _listed(e, 'run')):
+            if run is None:
+                ket = elem.run(ket)
+                continue
+            bit_of = _bits_of(ket.qubits)
+            bits = [b for gate, _ in run for b in _lookup(bit_of, gate.qubits)]
+            tensor = bk.apply_gates(ket.tensor, [kind for _, kind in run], bits)
+            ket = State(tensor, ket.qubits, ket.memory)
+        return ket
+
     def asgate(self) -> Gate:
-        """The circuit's unitary, composed on the GPU (circuits.py:111-118)."""
-        gate = identity_gate(self.qubits)
-        for elem in self.elements:
-            gate = elem.asgate() @ gate
-        return gate
+        """The circuit's unitary, composed on the GPU (circuits.py:111-118):
+        its gates act on the row axes of the identity."""
+        qubits = self.qubits
+        gate = None
+
+        def item(elem):
+            return _listed(elem, 'asgate') if type(elem).__matmul__ is Gate.__matmul__ else None
+        for run, elem in _runs(self.elements, item):
+            if run is None:
+                gate = elem.asgate() @ (identity_gate(qubits) if gate is None else gate)
+                continue
+            n = len(qubits)
+            bit_of = {q: b + n for q, b in _bits_of(qubits).items()}
+            bits = [b for g, _ in run for b in _lookup(bit_of, g.qubits)]
+            tensor = bk.identity_tensor(n) if gate is None else gate.tensor
+            gate = Gate(tensor=bk.apply_gates(tensor, [kind for _, kind in run], bits),
+                        qubits=qubits)
+        return identity_gate(qubits) if gate is None else gate
 
     def aschannel(self):
         """The circuit's superoperator: the identity channel on its qubits

@@ -118,7 +118,7 @@ __global__ __launch_bounds__(kBlock) void sparse_kernel(double2* out, const doub
 #pragma unroll
       for (int r = 0; r < D; ++r) {
         if (ALL || (a.active & (1u << r))) {
-          const double2 x = (a.has_phase & (1u << r)) ? cmul(a.ph[r], v[u][r]) : v[u][r];
+          const double2 x = (a.has_phase & (1u << r)) ? cmul_fma(a.ph[r], v[u][r]) : v[u][r];
           st_amp<NT>(out + base[u] + a.off[r], x);
         }
       }

@@ -90,6 +90,17 @@ __device__ __forceinline__ v2d cmul(const v2d a, const v2d b) {
   return r;
 }
 
+// cmul with its roundings spelled out, so that every kernel that applies a
+// gate's phases gives the same bits (which product of cmul the compiler fuses
+// differs from kernel to kernel).
+template <typename V>
+__device__ __forceinline__ V cmul_fma(const V a, const V b) {
+  V r;
+  r.x = fma(a.x, b.x, -(a.y * b.y));
+  r.y = fma(a.y, b.x, a.x * b.y);
+  return r;
+}
+
 // complex multiply-accumulate: acc += a * b
 __device__ __forceinline__ void cmac(double2& acc, const double2 a, const double2 b) {
   acc.x = fma(a.x, b.x, acc.x);

@@ -62,10 +62,9 @@ def _to_host_matrix(tensor):
     else:
         arr = np.asarray(tensor)
     arr = np.asarray(arr, dtype=np.complex128)
-    n = int(round(np.log2(arr.size)))
-    if 2 ** n != arr.size or n % 2:
+    k, odd = divmod(arr.size.bit_length() - 1, 2)
+    if arr.size != 4 ** k or odd:
         raise ValueError('Incompatibility between tensor and qubits')
-    k = n // 2
     return arr.reshape(2 ** k, 2 ** k)
 
 
@@ -85,7 +84,7 @@ class Gate(Operation):
             self._dev = dev.reshape([2] * n) if n else dev
         else:
             self._host = _to_host_matrix(tensor)
-            k = int(round(np.log2(self._host.shape[0])))
+            k = self._host.shape[0].bit_length() - 1
         if qubits is None:
             qubits = range(k)
         qubits = tuple(qubits)
