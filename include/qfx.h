@@ -353,8 +353,8 @@ int qfx_cut_counts(void* stream, void* out, int n, const void* edges, int m);
  * Circuit.run -> State.expectation(graph_cuts) (quantumflow/qaoa.py:22-81,
  * quantumflow/states.py:131-147) and the autograd gradient of
  * examples/qaoa_maxcut.py:53-64.  The host builds, per instance, a program
- * of tiled passes (tile bit set + stages); global pass k of all instances
- * runs between grid barriers.  Every array below is device memory. */
+ * of tiled passes (tile bit set + stages).  An instance's pass k starts when
+ * its pass k - 1 is done.  Every array below is device memory. */
 
 #define QFX_QAOA_MAX_LAYERS 16
 #define QFX_QAOA_MAX_STAGES 40
@@ -392,12 +392,11 @@ typedef struct {
   int32_t flags;      /* 1 load psi, 2 load lambda, 4 store psi, 8 store lambda */
   /* {type, layer, tile-bit mask}; types: 1 init |+>, 2 cost layer, 3 RX on
    * the mask, 4 <C>, 5 lambda = C psi, 6 adjoint RX, 7 adjoint cost layer,
-   * 8 cost layer then RX of the same layer (forward programs only; the
-   * phases ride in the first RX chunk; mask must be non-empty), 10 / 11 RX
-   * applied while the tile is loaded / stored (forward programs only; the
-   * pass's first stage with flag 1 / last stage with flag 4; the bits a
-   * thread holds in registers then, the 4 tile bits above log2(block), cost
-   * no LDS sweep, any others run as an LDS chunk) */
+   * 8 cost layer then RX of the same layer (forward programs only; mask must
+   * be non-empty), 10 / 11 RX as the pass's first stage with flag 1 / last
+   * stage with flag 4 (forward programs only).  The kernel keeps its tile in
+   * registers through all stages and runs 8 as its two parts and 10 / 11 as
+   * 3. */
   int32_t stage[QFX_QAOA_MAX_STAGES][3];
 } qfx_qaoa_pass;
 
@@ -412,7 +411,8 @@ typedef struct {
   const void* insts;      /* qfx_qaoa_inst[ninst] */
   const void* passes;     /* qfx_qaoa_pass[] */
   const void* items;      /* qfx_qaoa_item[], grouped by global pass */
-  const void* kstart;     /* int32[nk + 1]: items of global pass k */
+  const void* kstart;     /* int32[nk + 1]: items of global pass k; an item's
+                             instance has its earlier passes in earlier ones */
   const void* angles;     /* float64 */
   void* psi_pool;         /* complex128 */
   void* lam_pool;         /* complex128 (backward) */
@@ -426,21 +426,32 @@ typedef struct {
                              resets the first two and leaves the third, which
                              any grid-barrier timeout sets. */
   int32_t ninst, nk, width, mode, block, max_items_per_k;
-  int32_t tile_bits;      /* largest pass tile (LDS per workgroup: 2^tile_bits
-                             amplitudes, twice that backward); 0: 13 forward,
-                             12 backward.  Must be what qfx_qaoa_check
-                             accepted the program with. */
+  int32_t tile_bits;      /* largest pass tile (13-bit backward tiles take a
+                             CU each, all others half of one); 0: 13.  Must
+                             be what qfx_qaoa_check accepted the program
+                             with. */
   int32_t pad;
   void* timing;           /* NULL, or uint64 [timing_len]: per global pass k
                              and workgroup b, entries 2 (k grid + b) and +1
                              get the device wall clock when b starts pass k
-                             and when it reaches the barrier after it (entries
+                             and when it leaves it (entries
                              past timing_len are not written) */
   int64_t timing_len;
+  /* All three, or NULL: grid barriers between the global passes.  With them
+     every instance keeps at most 2^27 amplitudes, and nothing else may use
+     the workspace during the launch. */
+  void* tables;           /* complex128 workspace of the launch: counters in
+                             the first 32 + ninst entries, then from
+                             table_off[i] instance i's mixers and phases,
+                             p times (8 + (weighted ? 0 : nedges + 1)) */
+  const void* table_off;  /* int64[ninst] */
+  const void* item_need;  /* int32[items]: items of its instance that must be
+                             done before the item starts, all earlier in the
+                             list */
 } qfx_qaoa_args;
 
 /* Host-side validation of a program (host copies of the device arrays);
- * tile_bits as in qfx_qaoa_args (0: the mode's default). */
+ * tile_bits as in qfx_qaoa_args (0: 13). */
 int qfx_qaoa_check(const qfx_qaoa_inst* insts, int ninst,
                    const qfx_qaoa_pass* passes, int npasses,
                    const qfx_qaoa_item* items, const int* kstart, int nk,
@@ -448,14 +459,15 @@ int qfx_qaoa_check(const qfx_qaoa_inst* insts, int ninst,
                    int64_t cnt_pool_len, int64_t val_pool_len,
                    int64_t npartial, int mode, int tile_bits);
 
-/* Enqueue the program: a barrier reset, the persistent kernel (grid = the
- * workgroups that fit the device at once) and the per-instance reduction
- * into out.  Capturable into a HIP graph. */
+/* Enqueue the program: a kernel that resets the barrier and makes the tables,
+ * the persistent kernel (grid = the workgroups that fit the device at once;
+ * 512 lanes each, whatever `block` says) and the per-instance reduction into
+ * out.  Capturable into a HIP graph. */
 int qfx_qaoa_run(void* stream, const qfx_qaoa_args* args);
 
-/* After the stream completes: *failed = 1 if a grid barrier timed out in
+/* After the stream completes: *failed = 1 if a wait for other items timed out in
  * the last launch or in any earlier launch since the owner zeroed the
- * sticky flag.  A barrier times out after 10 s of device wall-clock time. */
+ * sticky flag.  A wait times out after 10 s of device wall-clock time. */
 int qfx_qaoa_status(const void* sync, int* failed);
 
 /* ---- MLP angle proposer kernels (fp32) ----------------------------------

@@ -14,10 +14,10 @@ the reference's plain gradient ascent for all instances at once.
 Program of one instance (built on the host by ``build_program``): the gate
 sequence H^n, [cost(l), RX(l) on every qubit] for l < p, then <C>, and in
 backward mode lambda = C psi followed by the stages undone in reverse.  It is
-split into passes over tile bit sets of at most T bits (13 forward, 12
-backward): the low 13 (12) bits, then the low 3 bits plus the next chunk of
+split into passes over tile bit sets of at most T bits (13 forward, 12 or 13
+backward): the low T bits, then the low 3 bits plus the next chunk of
 high bits, and so on; an RX stage on bits outside the current set closes the
-pass.  Instances with n <= T run as one pass entirely in LDS.
+pass.  Instances with n <= T run as one pass entirely in registers.
 """
 
 import ctypes
@@ -32,17 +32,23 @@ from . import backend as bk
 
 MODE_FORWARD, MODE_BACKWARD = 0, 1
 ST_INIT, ST_COST, ST_RX, ST_EXPECT, ST_MAKE_LAMBDA, ST_RX_ADJ, ST_COST_ADJ = 1, 2, 3, 4, 5, 6, 7
-# fused stage: cost layer l then RX layer l (the phases ride in the first
-# mixer chunk)
+# fused stage: cost layer l then RX layer l
 ST_COST_RX = 8
-# RX layer l on tile bits applied in registers while the tile is loaded
-# from / stored to HBM (the pass's first / last stage)
+# RX layer l on tile bits as the pass's first / last stage, beside the load /
+# store
 ST_RX_LOAD, ST_RX_STORE = 10, 11
-IO_BITS = 4               # tile bits above log2(block) a thread holds in registers
+IO_BITS = 4               # tile bits above log2(block) such a stage takes
 PF_LOAD_PSI, PF_LOAD_LAM, PF_STORE_PSI, PF_STORE_LAM = 1, 2, 4, 8
 MAX_LAYERS = 16
 MAX_STAGES = 40
 LOW_BITS = 3
+FLOW_KEPT = 2 ** 27       # kept amplitudes that qfx_qaoa_args.item_need allows
+# State of the instances whose passes are listed together: their passes follow
+# each other while it is still in the 256 MiB cache beside the cut tables.  104
+# values of 10 to 22 qubits (512 MiB of state): 64 MiB 1466 us, 96 1386, 128
+# 1204, 192 1196, 256 1268, all at once 1309; smaller groups run out of items.
+GROUP_BYTES = 192 * 2 ** 20
+TABLE_HEAD, MIXER = 32, 8  # entries of qfx_qaoa_args.tables
 
 
 class QaoaInst(ctypes.Structure):
@@ -70,7 +76,9 @@ class QaoaArgs(ctypes.Structure):
                [(nm, ctypes.c_int32) for nm in
                 ('ninst', 'nk', 'width', 'mode', 'block', 'max_items_per_k', 'tile_bits',
                  'pad')] + \
-               [('timing', ctypes.c_void_p), ('timing_len', ctypes.c_int64)]
+               [('timing', ctypes.c_void_p), ('timing_len', ctypes.c_int64),
+                ('tables', ctypes.c_void_p), ('table_off', ctypes.c_void_p),
+                ('item_need', ctypes.c_void_p)]
 
 
 def tile_sets(n, T, low=None):
@@ -116,12 +124,51 @@ def use_mirror(n, T):
     return n >= T + 2 and T >= 2
 
 
+def batch_bits(ns, mode, T):
+    """Tile bits of each instance's passes in a batch of T tile bits: T, but in
+    a backward batch of 12 those of 13 and of 18 qubits and more take 13 (one
+    pass for 13, two passes a layer and not four for 23 and 24, longer runs
+    for the others) if that gives work to 192 of the 256 workgroups of 13-bit
+    tiles that run at once; 12-bit tiles run 512.  Measured, 12 / 13 bits, 8
+    layers: 128 instances of 13 qubits 243 / 207 us, 16 of 18 609 / 594, 8 of
+    19 835 / 635, 1 of 22 977 / 681, 1 of 23 2980 / 1475, 1 of 24 6468 / 3347;
+    but 4 of 19 371 / 444, 1 of 20 286 / 411, 1 of 21 413 / 526, and 64 of 16
+    414 / 499."""
+    if mode == MODE_BACKWARD and T == 12:
+        gain = [n == 13 or n >= 18 for n in ns]
+        if sum(2 ** max(n - 14, 0) for n, g in zip(ns, gain) if g) >= 192:
+            return [13 if g else T for g in gain]
+    return [T] * len(ns)
+
+
+def instance_groups(state_bytes, limit):
+    """Instances in the order their items are listed, by the state they keep
+    and as many to a group as keep at most `limit` bytes (at least one)."""
+    order = sorted(range(len(state_bytes)), key=lambda i: state_bytes[i])
+    groups, held = [], math.inf
+    for i in order:
+        if held + state_bytes[i] > limit:
+            groups.append([])
+            held = 0
+        groups[-1].append(i)
+        held += state_bytes[i]
+    return groups
+
+
+def by_xcd(items):
+    """Every 64 items in the order that gives 8 neighbouring tiles to one of
+    the 8 XCDs, to which items go in turn: a tile that holds only part of each
+    128-byte line shares them with its neighbours, through one L2.  24 qubits
+    backward, tiles of 32-byte runs: 3.34 ms, in plain order 3.70."""
+    whole = len(items) // 64 * 64
+    return [items[c + (q % 8) * 8 + q // 8] for c in range(0, whole, 64) for q in range(64)] \
+        + items[whole:]
+
+
 def fuse_stages(stages):
     """Merge a cost stage into the mixer stage of the same layer that follows
-    it in a pass: (COST l, RX l) -> COST_RX l.  The kernel then applies the
-    phases inside the first RX chunk instead of in a sweep of their own.
-    The adjoint stages stay separate: with lambda and psi both in registers,
-    a fused adjoint chunk measured slower than the two sweeps."""
+    it in a pass: (COST l, RX l) -> COST_RX l.  The adjoint stages stay
+    separate."""
     out = []
     for st in stages:
         typ, layer, bits = st
@@ -135,13 +182,10 @@ def fuse_stages(stages):
 
 
 def io_stages(tset, stages, flags, block):
-    """Move RX bits that a thread holds in registers during the tile's HBM
-    load or store out of the pass's first or last mixer stage.  Thread t
-    owns tile elements t + k*block and holds 2^IO_BITS consecutive k at a
-    time, so the tile bits log2(block) .. +IO_BITS-1 pair elements of one
-    thread: RX on them needs no LDS sweep.  The first stage gives up such bits to ST_RX_LOAD when the
+    """Split the tile bits log2(block) .. +IO_BITS-1 off the pass's first or
+    last mixer stage: the first stage gives them up to ST_RX_LOAD when the
     pass loads the state; the last to ST_RX_STORE when it stores it.  A
-    stage keeps at least one bit (a fused cost stage needs its chunk)."""
+    stage keeps at least one bit."""
     lb = block.bit_length() - 1
     kset = {b for j, b in enumerate(tset) if lb <= j < lb + IO_BITS}
     stages = list(stages)
@@ -162,12 +206,10 @@ def io_stages(tset, stages, flags, block):
 def build_program(n, p, mode, T, fuse=True, block=512, mirror=False):
     """Passes of one instance: list of (tile bits, [(stage, layer, global bit
     set)], flags).  With `fuse`, forward-mode programs merge each cost stage
-    into the mixer stage of its layer (fuse_stages) and apply RX bits held
-    in registers during the tile's load and store (io_stages, for
-    `block`-thread workgroups).  Backward programs keep their cost stages
-    separate: their 12-bit tiles leave a 4-bit chunk only 256 groups, half
-    of a 512-thread workgroup, and the fused stage measured slower there
-    than the separate sweep."""
+    into the mixer stage of its layer (fuse_stages) and split RX bits off
+    beside the tile's load and store (io_stages); backward programs keep
+    their stages separate.  The kernel holds its tile in registers through
+    all of them, so all forms do the same work."""
     allbits = frozenset(range(n))
     seq = [(ST_INIT, 0, None)]
     for l in range(p):
@@ -222,7 +264,7 @@ def program_bytes(n, p, mode, T, block=512, mirror=False, weighted=False, fuse=T
     """Algorithmic HBM bytes of one instance's program: (state, cut table).
     State: 16 B per kept amplitude (2^n, or 2^(n-1) for a mirror instance)
     for every load and store of psi and lambda a pass makes (a one-pass
-    instance keeps its state in LDS).  Cut table: 2 B (unit weights) or 8 B
+    instance keeps its state in registers).  Cut table: 2 B (unit weights) or 8 B
     per kept amplitude for every stage that reads the cost of each index
     (cost layers, fused cost-mixer stages, <C>, lambda = C psi, adjoint cost
     layers)."""
@@ -281,19 +323,22 @@ class QAOABatch:
         bk.stream_handle()                          # initialise the device
         ninst = len(self.graphs)
         insts = (QaoaInst * ninst)()
-        pass_list, items_by_k = [], []
+        pass_list, progs = [], []
         psi_len = lam_len = 0
+        state_bytes = []                  # kept in the pools, per instance
+        most_kept = 0
         cnt_len = val_len = 0
         slot = 0
         single_max = 1
-        self.n = []
         self.maxcut = np.zeros(ninst)
         cut_jobs = []
-        for i, g in enumerate(self.graphs):
-            n, edges, w, weighted = graph_arrays(g)
-            self.n.append(n)
-            mir = bool(mirror) and use_mirror(n, T)
-            prog = build_program(n, p, mode, T, fuse, block, mirror=mir)
+        arrays = [graph_arrays(g) for g in self.graphs]
+        self.n = [x[0] for x in arrays]
+        self._bits = batch_bits(self.n, mode, T)
+        for i, (n, edges, w, weighted) in enumerate(arrays):
+            width = self._bits[i]
+            mir = bool(mirror) and use_mirror(n, width)
+            prog = build_program(n, p, mode, width, fuse, block, mirror=mir)
             inst = insts[i]
             inst.n, inst.p, inst.weighted, inst.nedges = n, p, int(weighted), len(edges)
             inst.mirror = int(mir)
@@ -318,6 +363,9 @@ class QAOABatch:
                 single_max = max(single_max, 2 ** n)
             inst.angle_off = 2 * p * i
             inst.slot0 = slot
+            progs.append([])
+            most_kept = max(most_kept, kept)
+            state_bytes.append((16 if mode == MODE_FORWARD else 32) * kept if len(prog) > 1 else 0)
             for q, (tset, stages, flags) in enumerate(prog):
                 ps = QaoaPass()
                 ps.T = len(tset)
@@ -338,27 +386,28 @@ class QAOABatch:
                 ps.flags = flags
                 pidx = len(pass_list)
                 pass_list.append(ps)
-                while len(items_by_k) <= q:
-                    items_by_k.append([])
                 # a mirror instance's items: tiles whose highest non-tile bit is clear
-                for t in range(2 ** (n - ps.T - (1 if mir else 0))):
-                    items_by_k[q].append((i, pidx, t, slot if accum else -1, 2 ** n))
-                    if accum:
-                        slot += 1
+                tiles = 2 ** (n - ps.T - (1 if mir else 0))
+                progs[i].append((pidx, tiles, slot if accum else -1))
+                if accum:
+                    slot += tiles
             inst.nslots = slot - inst.slot0
         self.dummy_slot = slot            # items without a reduction write here
         nslots = slot + 1
-        # global pass k: single-pass (whole-instance) items first, then big tiles
-        items, kstart = [], [0]
-        for k, lst in enumerate(items_by_k):
-            lst.sort(key=lambda x: (-(pass_list[x[1]].T == self.n[x[0]]) * x[4], x[0], x[2]))
-            for (i, pidx, t, sl, _) in lst:
-                it = QaoaItem()
-                it.inst, it.pass_, it.tile = i, pidx, t
-                it.partial = sl if sl >= 0 else self.dummy_slot
-                items.append(it)
-            kstart.append(len(items))
-        self.nk = len(items_by_k)
+        flow = most_kept <= FLOW_KEPT
+        items, kstart, need = [], [0], []
+        for members in instance_groups(state_bytes, GROUP_BYTES if flow else math.inf):
+            for q in range(max(len(progs[i]) for i in members)):
+                todo = [(i, progs[i][q], t) for i in members if q < len(progs[i])
+                        for t in range(progs[i][q][1])]
+                for i, (pidx, tiles, sl), t in by_xcd(todo):
+                    it = QaoaItem()
+                    it.inst, it.pass_, it.tile = i, pidx, t
+                    it.partial = sl + t if sl >= 0 else self.dummy_slot
+                    items.append(it)
+                    need.append(q * tiles)
+                kstart.append(len(items))
+        self.nk = len(kstart) - 1
         self.nitems = len(items)
         psi_len = max(psi_len, single_max)
         lam_len = max(lam_len, single_max)
@@ -371,7 +420,8 @@ class QAOABatch:
                                          self.nk, self.width, psi_len,
                                          lam_len if mode == MODE_BACKWARD else 0,
                                          max(cnt_len, 1) if cnt_len else 0,
-                                         max(val_len, 1) if val_len else 0, nslots, mode, T),
+                                         max(val_len, 1) if val_len else 0, nslots, mode,
+                                         max(ps.T for ps in pass_list)),
                       'qfx_qaoa_check')
 
         def up(arr):
@@ -389,6 +439,12 @@ class QAOABatch:
         self.out = torch.zeros(ninst * self.width, dtype=torch.float64, device=dev)
         self.sync = torch.zeros(4, dtype=torch.int32, device=dev)
         self.angles = torch.zeros(ninst * 2 * p, dtype=torch.float64, device=dev)
+        # every launch's counters, mixers and cost phases (qfx_qaoa_args.tables)
+        head = TABLE_HEAD + ninst
+        sizes = [p * (MIXER + (0 if i.weighted else i.nedges + 1)) for i in insts]
+        self._table_off = torch.tensor(head + np.concatenate([[0], np.cumsum(sizes)[:-1]]),
+                                       dtype=torch.int64, device=dev)
+        self._tables = torch.empty(head + sum(sizes), dtype=torch.complex128, device=dev)
         # cut tables on the GPU
         s = bk.stream_handle()
         for (n, edges, w, weighted, off) in cut_jobs:
@@ -411,22 +467,27 @@ class QAOABatch:
             self._items.data_ptr()
         a.kstart, a.angles = self._kstart.data_ptr(), self.angles.data_ptr()
         a.psi_pool, a.lam_pool = self.psi_pool.data_ptr(), self.lam_pool.data_ptr()
-        a.cnt_pool, a.val_pool = self.cnt_pool.data_ptr(), self.val_pool.data_ptr()
+        a.cnt_pool = self.cnt_pool.data_ptr()
+        a.val_pool = self.val_pool.data_ptr() if val_len else None
         a.partials, a.out, a.sync = self.partials.data_ptr(), self.out.data_ptr(), \
             self.sync.data_ptr()
         a.ninst, a.nk, a.width, a.mode, a.block = ninst, self.nk, self.width, mode, block
         a.max_items_per_k = max(kstart[k + 1] - kstart[k] for k in range(self.nk))
-        a.tile_bits = T
+        a.tile_bits = max(ps.T for ps in pass_list)
+        self._need = torch.tensor(need, dtype=torch.int32, device=dev)
+        if flow:
+            a.tables, a.table_off = self._tables.data_ptr(), self._table_off.data_ptr()
+            a.item_need = self._need.data_ptr()
         self._graph = None
 
     def algorithmic_bytes(self):
         """(state bytes, cut-table bytes) one launch moves, summed over the
         instances (program_bytes)."""
         st = ct = 0
-        for g, n in zip(self.graphs, self.n):
+        for g, n, width in zip(self.graphs, self.n, self._bits):
             weighted = graph_arrays(g)[3]
-            a, b = program_bytes(n, self.p, self.mode, self.T, self.block,
-                                 self._mirror and use_mirror(n, self.T), weighted, self._fuse)
+            a, b = program_bytes(n, self.p, self.mode, width, self.block,
+                                 self._mirror and use_mirror(n, width), weighted, self._fuse)
             st += a
             ct += b
         return st, ct
@@ -476,11 +537,10 @@ class QAOABatch:
 
     def pass_times(self, max_grid=4096):
         """One launch with the kernel's wall-clock stamps on.  Per global pass
-        k: its items, its span (first workgroup start to last arrival at the
-        barrier after it) and the mean and largest time a workgroup spent on
-        its items, in microseconds (device wall clock, qfx_init's rate).
-        The gap between span and mean busy time is barrier wait and load
-        imbalance."""
+        k: its items, its span (first workgroup start to last end) and the mean
+        and largest time a workgroup spent on its items and on waiting for the
+        items before them, in microseconds (device wall clock, qfx_init's
+        rate).  Passes overlap: the next one starts where its items can."""
         dev = bk.DEVICE
         khz = bk.device_props()[7]
         if khz <= 0:
@@ -528,7 +588,7 @@ class QAOABatch:
 
 
 def raise_if_failed(flag):
-    """The engine's status word: nonzero means a grid barrier gave up, and
+    """The engine's status word: nonzero means a wait for other items gave up, and
     the values and gradients of that launch are partial."""
     if flag:
         raise RuntimeError('qaoa engine: grid barrier timed out; results are partial')

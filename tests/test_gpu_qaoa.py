@@ -331,3 +331,89 @@ def test_mirror_half_state_matches_full_state(E, mode):
     i = 3
     ref = O.qaoa_expectation_fast(len(graphs[i]), list(graphs[i].edges()), beta[i], gamma[i])
     assert abs(v1.cpu().numpy()[i] - ref) <= 1e-10
+
+
+def _plain(n, edges, w, beta, gamma, grad):
+    """Value and gradient in 64 bits, one gate at a time."""
+    import torch
+    z = torch.arange(2 ** n)
+    c = torch.zeros(2 ** n, dtype=torch.float64)
+    for (u, v), x in zip(edges, w):
+        c += x * ((z >> (n - 1 - u) ^ z >> (n - 1 - v)) & 1).double()
+
+    def rx(psi, t):
+        for j in range(n):
+            v = psi.view(-1, 2, 2 ** j)
+            psi = (np.cos(t / 2) * v - 1j * np.sin(t / 2) * v.flip(1)).reshape(-1)
+        return psi
+    ph = [torch.exp(1j * g * (sum(w) / 2 - c)) for g in gamma]
+    psi = torch.full((2 ** n,), 2.0 ** (-n / 2), dtype=torch.complex128)
+    for l, b in enumerate(beta):
+        psi = rx(psi * ph[l], b)
+    value = torch.sum(psi.abs() ** 2 * c).item()
+    if not grad:
+        return value, None
+    lam, db, dg = psi * c, [], []
+    for l in reversed(range(len(beta))):
+        db.insert(0, sum(torch.vdot(lam, psi.view(-1, 2, 2 ** j).flip(1).reshape(-1)).imag.item()
+                         for j in range(n)))
+        psi, lam = rx(psi, -beta[l]), rx(lam, -beta[l])
+        dg.insert(0, (2 * torch.vdot(lam, c * psi) - sum(w) * torch.vdot(lam, psi)).imag.item())
+        psi, lam = psi * ph[l].conj(), lam * ph[l].conj()
+    return value, np.array(db + dg)
+
+
+@pytest.mark.parametrize("barriers", [False, True])
+@pytest.mark.parametrize("mode,T", [(0, 6), (0, 9), (0, 10), (0, 11), (0, 12), (0, 13),
+                                    (1, 6), (1, 9), (1, 10), (1, 11), (1, 12)])
+def test_tile_widths_angles_and_waits(E, mode, T, barriers, monkeypatch):
+    """Every tile width (registers a lane, idle lanes, wave bits with and
+    without the exchange), instances below, at and above it, whole and
+    mirrored, unit and weighted, mixer angles on both sides of the flip and at
+    its edges; by item waits in groups of one instance and by grid barriers.
+    An amplitude gathers about 3 roundings of 2^-53 a qubit and layer, so
+    values and gradient terms, sums of |E| C-weighted amplitudes, stay within
+    3 * 14 * 4 * 2^-53 |E|^2 < 6e-11 (|E| < 56)."""
+    monkeypatch.setattr(E, 'GROUP_BYTES', 1)
+    rng = np.random.default_rng(100 * mode + T)
+    sizes = sorted({1, 2, 5, T - 1, T, T + 1, min(T + 3, 14)})
+    graphs = [er(n, 0.6, 7 * n + T) for n in sizes] + [er(T + 1, 0.6, 3)]
+    for u, v in graphs[-1].edges():
+        graphs[-1][u][v]['weight'] = float(rng.uniform(0.1, 2.0))
+    beta = rng.uniform(-7, 7, size=(len(graphs), 4))
+    beta[:, 1] = rng.choice([0.0, np.pi / 2, -np.pi / 2, np.pi, 2 * np.pi], size=len(graphs))
+    gamma = rng.uniform(-3, 3, size=(len(graphs), 4))
+    for mirror in (True, False):
+        b = E.QAOABatch(graphs, 4, mode=mode, tile_bits=T, mirror=mirror)
+        if barriers:
+            b._args.tables = b._args.item_need = None
+        for _ in range(2):                        # a launch leaves nothing behind
+            val, grad = b.evaluate(beta, gamma)
+            b.check()
+            for i, g in enumerate(graphs):
+                w = [g[u][v].get('weight', 1.0) for u, v in g.edges()]
+                v, gr = _plain(len(g), list(g.edges()), w, beta[i], gamma[i], mode == 1)
+                assert abs(val[i].item() - v) <= 6e-11, (len(g), mirror)
+                if mode == 1:
+                    assert np.max(np.abs(grad[i].cpu().numpy() - gr)) <= 6e-11, (len(g), mirror)
+
+
+def test_wide_backward_tiles(E, monkeypatch):
+    """13-bit backward tiles against 12-bit ones: 13 qubits in one pass, 18
+    in two sets, weighted ones beside them; within 8 * 18 * 3 * 2^-53 |E|^2
+    of each other (|E| < 64: 2e-10)."""
+    rng = np.random.default_rng(4)
+    graphs = [er(n, 0.4, n) for n in [13] * 20 + [16, 18, 13]]
+    for u, v in graphs[-1].edges():
+        graphs[-1][u][v]['weight'] = float(rng.uniform(0.1, 2.0))
+    beta = rng.uniform(-4, 4, size=(len(graphs), 3))
+    gamma = rng.uniform(-3, 3, size=(len(graphs), 3))
+    res = []
+    for bits in ([12] * len(graphs), [13 if len(g) in (13, 18) else 12 for g in graphs]):
+        monkeypatch.setattr(E, 'batch_bits', lambda ns, mode, T: bits)
+        b = E.QAOABatch(graphs, 3, mode=E.MODE_BACKWARD)
+        val, grad = b.evaluate(beta, gamma)
+        b.check()
+        res.append((val.cpu().numpy().copy(), grad.cpu().numpy().copy()))
+    assert np.max(np.abs(res[0][0] - res[1][0])) <= 2e-10
+    assert np.max(np.abs(res[0][1] - res[1][1])) <= 2e-10
