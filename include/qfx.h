@@ -302,6 +302,8 @@ typedef struct {
                               phase loading straight from HBM (no LDS round
                               trip before it); needs 2^tile_bits == 16 * block,
                               block <= 512; combines with QFX_TILE_REG_IO */
+#define QFX_TILE_PHASES 32 /* flags: with QFX_TILE_REG_IN, a pass of two or more
+                              ops, all register phases */
 
 /* Fills the derived `lds` words of every register phase in ops[0..nops-1]
  * (host array) from its tile bits and maps; zeroes them for other kinds.

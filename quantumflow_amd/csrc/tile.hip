@@ -224,13 +224,13 @@ constexpr int kCxFlip = 1 << 10;           // SUB_CX code: controls compared thr
 constexpr int kRecType = 255;
 
 // 1-qubit sub-ops walk the 8 register pairs (r, r | 1 << A); a scheduling
-// fence after the first four keeps half of the results in flight at a time
-// (all eight would push the kernel past 256 VGPRs, i.e. below two waves per
-// SIMD).
+// fence after every F keeps only their results in flight at a time: four
+// where two waves share a SIMD (all eight would push the kernel past 256
+// VGPRs, i.e. below that), one where three do.
 template <int A>
 constexpr int pair_lo(int p) { return ((p >> A) << (A + 1)) | (p & ((1 << A) - 1)); }
 
-template <int A>
+template <int A, int F>
 __device__ __forceinline__ void sub_d1(v2d (&v)[kRegs], const v2d m0, const v2d m1, const v2d m2,
                                        const v2d m3) {
 #pragma unroll
@@ -244,11 +244,11 @@ __device__ __forceinline__ void sub_d1(v2d (&v)[kRegs], const v2d m0, const v2d 
     cmac(b, m3, y);
     v[r] = a;
     v[r | (1 << A)] = b;
-    if (p == kRegs / 4 - 1) __builtin_amdgcn_sched_barrier(0);
+    if (p % F == F - 1 && p != kRegs / 2 - 1) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-template <int A>
+template <int A, int F>
 __device__ __forceinline__ void sub_d1r(v2d (&v)[kRegs], const double m0, const double m1,
                                         const double m2, const double m3) {
 #pragma unroll
@@ -257,12 +257,12 @@ __device__ __forceinline__ void sub_d1r(v2d (&v)[kRegs], const double m0, const 
     const v2d x = v[r], y = v[r | (1 << A)];
     v[r] = v2d{fma(m0, x.x, m1 * y.x), fma(m0, x.y, m1 * y.y)};
     v[r | (1 << A)] = v2d{fma(m2, x.x, m3 * y.x), fma(m2, x.y, m3 * y.y)};
-    if (p == kRegs / 4 - 1) __builtin_amdgcn_sched_barrier(0);
+    if (p % F == F - 1 && p != kRegs / 2 - 1) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
 // [[c0, i s0], [i s1, c1]]
-template <int A>
+template <int A, int F>
 __device__ __forceinline__ void sub_d1x(v2d (&v)[kRegs], const double c0, const double s0,
                                         const double s1, const double c1) {
 #pragma unroll
@@ -271,7 +271,7 @@ __device__ __forceinline__ void sub_d1x(v2d (&v)[kRegs], const double c0, const 
     const v2d x = v[r], y = v[r | (1 << A)];
     v[r] = v2d{fma(c0, x.x, -s0 * y.y), fma(c0, x.y, s0 * y.x)};
     v[r | (1 << A)] = v2d{fma(c1, y.x, -s1 * x.y), fma(c1, y.y, s1 * x.x)};
-    if (p == kRegs / 4 - 1) __builtin_amdgcn_sched_barrier(0);
+    if (p % F == F - 1 && p != kRegs / 2 - 1) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -425,6 +425,7 @@ __device__ __forceinline__ void sub_cx(v2d (&v)[kRegs], unsigned cm, unsigned cv
 // type and code below is one of the listed cases; the unreachable defaults
 // let the dispatch drop its do-nothing path, which would otherwise copy all
 // 16 register amplitudes on every sub-op.
+template <int F>
 __device__ __forceinline__ void apply_sub(v2d (&v)[kRegs], const int4 sub, const v2d* coef,
                                           uint64_t gbase, unsigned egrp, unsigned& fm) {
   const int type = sub.x, code = sub.y;
@@ -434,10 +435,10 @@ __device__ __forceinline__ void apply_sub(v2d (&v)[kRegs], const int4 sub, const
       // flagged: 8 coefficients, X m X in the second four for flipped lanes
       const v2d* mm = m + d1_offset(sub, fm, gbase, egrp);
       switch (code & 3) {
-        case 0: sub_d1<0>(v, mm[0], mm[1], mm[2], mm[3]); break;
-        case 1: sub_d1<1>(v, mm[0], mm[1], mm[2], mm[3]); break;
-        case 2: sub_d1<2>(v, mm[0], mm[1], mm[2], mm[3]); break;
-        case 3: sub_d1<3>(v, mm[0], mm[1], mm[2], mm[3]); break;
+        case 0: sub_d1<0, F>(v, mm[0], mm[1], mm[2], mm[3]); break;
+        case 1: sub_d1<1, F>(v, mm[0], mm[1], mm[2], mm[3]); break;
+        case 2: sub_d1<2, F>(v, mm[0], mm[1], mm[2], mm[3]); break;
+        case 3: sub_d1<3, F>(v, mm[0], mm[1], mm[2], mm[3]); break;
         default: __builtin_unreachable();
       }
       break;
@@ -445,10 +446,10 @@ __device__ __forceinline__ void apply_sub(v2d (&v)[kRegs], const int4 sub, const
     case SUB_D1R: {
       const v2d* mm = m + d1_offset(sub, fm, gbase, egrp);
       switch (code & 3) {
-        case 0: sub_d1r<0>(v, mm[0].x, mm[1].x, mm[2].x, mm[3].x); break;
-        case 1: sub_d1r<1>(v, mm[0].x, mm[1].x, mm[2].x, mm[3].x); break;
-        case 2: sub_d1r<2>(v, mm[0].x, mm[1].x, mm[2].x, mm[3].x); break;
-        case 3: sub_d1r<3>(v, mm[0].x, mm[1].x, mm[2].x, mm[3].x); break;
+        case 0: sub_d1r<0, F>(v, mm[0].x, mm[1].x, mm[2].x, mm[3].x); break;
+        case 1: sub_d1r<1, F>(v, mm[0].x, mm[1].x, mm[2].x, mm[3].x); break;
+        case 2: sub_d1r<2, F>(v, mm[0].x, mm[1].x, mm[2].x, mm[3].x); break;
+        case 3: sub_d1r<3, F>(v, mm[0].x, mm[1].x, mm[2].x, mm[3].x); break;
         default: __builtin_unreachable();
       }
       break;
@@ -456,10 +457,10 @@ __device__ __forceinline__ void apply_sub(v2d (&v)[kRegs], const int4 sub, const
     case SUB_D1X: {
       const v2d* mm = m + d1_offset(sub, fm, gbase, egrp);
       switch (code & 3) {
-        case 0: sub_d1x<0>(v, mm[0].x, mm[1].y, mm[2].y, mm[3].x); break;
-        case 1: sub_d1x<1>(v, mm[0].x, mm[1].y, mm[2].y, mm[3].x); break;
-        case 2: sub_d1x<2>(v, mm[0].x, mm[1].y, mm[2].y, mm[3].x); break;
-        case 3: sub_d1x<3>(v, mm[0].x, mm[1].y, mm[2].y, mm[3].x); break;
+        case 0: sub_d1x<0, F>(v, mm[0].x, mm[1].y, mm[2].y, mm[3].x); break;
+        case 1: sub_d1x<1, F>(v, mm[0].x, mm[1].y, mm[2].y, mm[3].x); break;
+        case 2: sub_d1x<2, F>(v, mm[0].x, mm[1].y, mm[2].y, mm[3].x); break;
+        case 3: sub_d1x<3, F>(v, mm[0].x, mm[1].y, mm[2].y, mm[3].x); break;
         default: __builtin_unreachable();
       }
       break;
@@ -580,6 +581,7 @@ __device__ __forceinline__ unsigned phase_lb(const qfx_tile_op& op, unsigned g) 
 }
 
 // Returns the lane's flip mask, which the phase's store applies.
+template <int F = kRegs / 4>
 __device__ __forceinline__ unsigned run_subs(v2d (&v)[kRegs], const qfx_tile_op& op,
                                              const v2d* coef, const int* __restrict__ subs,
                                              uint64_t gbase, unsigned egrp) {
@@ -604,12 +606,12 @@ __device__ __forceinline__ unsigned run_subs(v2d (&v)[kRegs], const qfx_tile_op&
     int4 cur = next;
     next = rec[i + 1 < nsub ? i + 1 : i];
     flips(cur);
-    apply_sub(v, cur, coef, gbase, egrp, fm);
+    apply_sub<F>(v, cur, coef, gbase, egrp, fm);
     if (i + 1 < nsub) {
       int4 cur2 = next;
       next = rec[i + 2 < nsub ? i + 2 : i + 1];
       flips(cur2);
-      apply_sub(v, cur2, coef, gbase, egrp, fm);
+      apply_sub<F>(v, cur2, coef, gbase, egrp, fm);
     }
   }
   return fm;
@@ -1229,6 +1231,112 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) void ti
   }
 }
 
+// ---- register-phase passes three waves to a SIMD --------------------------
+// A pass of register phases alone holds its tile in registers from load to
+// store, so LDS only carries it from one phase to the next: the real parts,
+// then the imaginary ones, through 8 bytes an amplitude.  With half the LDS and
+// no next tile beside its own (150 registers a lane) three workgroups share a
+// CU where tile_rin_kernel has two.  Its passes spend 42% of their cycles in
+// vector instructions and the rest on waits for scalar dispatch, LDS and
+// memory, which the third wave fills: 28 qubits, 25 sub-ops in 3 to 5 phases,
+// 2.66 -> 2.46 ms a pass (8 GiB of traffic, 1.8 ms at a copy's rate).  Four
+// (128 registers) spilled: 5.6 to 6.6 ms.
+typedef __attribute__((address_space(3))) double double_lds;
+
+__device__ __forceinline__ double_lds* lds_double(unsigned a) {
+  return (double_lds*)(size_t)a;
+}
+
+// From the slots of store bases `sa` (tree sb) to those of load bases `la`
+// (tree lb), all in bytes of the 16-byte layout.
+__device__ __forceinline__ void phase_exchange(v2d (&v)[kRegs], unsigned sa,
+                                               const unsigned (&sb)[4], unsigned la,
+                                               const unsigned (&lb)[4]) {
+  unsigned s2[4], l2[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    s2[j] = sb[j] >> 1;
+    l2[j] = lb[j] >> 1;
+  }
+#pragma unroll
+  for (int part = 0; part < 2; ++part) {
+    __syncthreads();
+    {
+      unsigned a[kRegs];
+      xor_tree(a, sa >> 1, s2);
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) *lds_double(a[r]) = v[r][part];
+    }
+    __syncthreads();
+    {
+      unsigned a[kRegs];
+      xor_tree(a, la >> 1, l2);
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) v[r][part] = *lds_double(a[r]);
+    }
+  }
+}
+
+template <int BS, int LB, bool REG_OUT>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(3))) void tile_phase_kernel(
+    v2d* state, TilePos pos, const qfx_tile_op* __restrict__ ops, int nops,
+    const v2d* __restrict__ coef, int ncoef, const int* __restrict__ srcs, uint32_t ntiles) {
+  constexpr int T = LB + kRegBits;
+  extern __shared__ v2d lds[];
+  const int tid = threadIdx.x;
+  const v2d* cf = stage_coef<BS>(lds, T - 1, coef, ncoef);
+  const uint64_t f_lane = tile_state_off(phase_lb(ops[0], (unsigned)tid), T, pos.s);
+  const PhaseGlobal fg = phase_global(ops[0], ops[0].phase, T, pos.s);
+  uint64_t soff = 0;                // where the lane stores, without REG_OUT
+#pragma unroll
+  for (int j = 0; j < LB; ++j) soff |= (uint64_t)((tid >> j) & 1) << pos.d[j];
+  __syncthreads();                  // staged coefficients
+  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    uint64_t base = tile;
+#pragma unroll
+    for (int j = 0; j < T; ++j) {
+      const int b = pos.s[j];
+      base = ((base >> b) << (b + 1)) | (base & (((uint64_t)1 << b) - 1));
+    }
+    // opaque: the 16 addresses made of each would be kept across the loop
+    uint64_t from = f_lane;
+    unsigned lane = tid;
+    asm("" : "+v"(from), "+v"(lane));
+    v2d v[kRegs];
+    phase_gload(v, state + base + from, fg);
+    for (int i = 0;; ++i) {
+      const qfx_tile_op& op = ops[i];
+      const unsigned egrp = phase_lb(op, lane);
+      const unsigned fm = run_subs<1>(v, op, cf, srcs, base, egrp);
+      if (i + 1 == nops) {
+        if constexpr (REG_OUT) {
+          phase_gstore(v, state + base + tile_state_off(egrp, T, pos.d),
+                       phase_global(op, op.active, T, pos.d), fm);
+        } else {
+          // to lane tid's amplitudes tid + r * BS
+          uint64_t to = soff;
+          asm volatile("" : "+v"(to), "+v"(lane));
+          const PhaseLds p = phase_lds(op);
+          const unsigned out[4] = {sw(BS) << 4, sw(2 * BS) << 4, sw(4 * BS) << 4, sw(8 * BS) << 4};
+          phase_exchange(v, (sw(egrp) << 4) ^ p.sc ^ flip_off(fm, p.s), p.s, sw(lane) << 4, out);
+          uint64_t h[4], a[kRegs];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) h[j] = (uint64_t)1 << pos.d[LB + j];
+          xor_tree(a, to, h);
+          v2d* q = state + base;
+#pragma unroll
+          for (int r = 0; r < kRegs; ++r) st_stream(q + a[r], v[r]);
+        }
+        break;
+      }
+      const qfx_tile_op& nx = ops[i + 1];
+      const PhaseLds p = phase_lds(op), q = phase_lds(nx);
+      phase_exchange(v, (sw(egrp) << 4) ^ p.sc ^ flip_off(fm, p.s), p.s,
+                     (sw(phase_lb(nx, lane)) << 4) ^ q.lc, q.l);
+    }
+  }
+}
+
 // Register phases address LDS by absolute byte offsets (lds_byte), valid
 // only when the kernel's dynamic LDS array starts at address 0, i.e. the
 // kernel has no static LDS; also raises the dynamic LDS limit.
@@ -1279,7 +1387,7 @@ int kernel_grid(const void* fn, const char* name, int block, size_t lds, int* gr
 template <int BS, int LB, bool WIDE, bool MF>
 int launch_pass(hipStream_t s, v2d* state, int n, int T, const TilePos& pos,
                 const qfx_tile_op* ops, int nops, const v2d* coef, int ncoef, const int* srcs,
-                bool persistent, bool reg_io, bool reg_in) {
+                bool persistent, bool reg_io, bool reg_in, bool phases) {
   constexpr bool kStage = !WIDE && !MF;
   const size_t lds = sizeof(v2d) * ((size_t(1) << T) + (kStage ? ncoef : 0));
   // occupancy (persistent grid size) for the largest staged table
@@ -1287,6 +1395,30 @@ int launch_pass(hipStream_t s, v2d* state, int n, int T, const TilePos& pos,
   const uint64_t tiles = (uint64_t)1 << (n - T);
   int grid = 0;
   int rc = QFX_OK;
+  // Passes of register phases alone, once the tiles fill the larger grid;
+  // fewer run as well two to a CU with the next tile in flight.  The same 40
+  // layers of gates, three / two to a CU: 22 qubits 484 / 562 us, 23 1054 /
+  // 1138, 25 4022 / 4318, 28 35.1 / 37.0 ms.  Only blocks of 256: one of 512
+  // would leave two waves to a SIMD, without the prefetch.
+  if constexpr (!WIDE && !MF && BS == 256) {
+    if (phases) {
+      // the coefficients in one of two sizes, so that few grids are asked for
+      const size_t want = sizeof(v2d) * ((size_t(1) << (T - 1)) + (ncoef <= 512 ? 512 : kMaxStaged));
+      const void* fn = reg_io ? (const void*)tile_phase_kernel<BS, LB, true>
+                              : (const void*)tile_phase_kernel<BS, LB, false>;
+      rc = kernel_grid(fn, "tile_phase_kernel", BS, want, &grid);
+      if (rc) return rc;
+      if (tiles >= (uint64_t)grid) {
+        if (reg_io)
+          hipLaunchKernelGGL((tile_phase_kernel<BS, LB, true>), dim3((unsigned)grid), dim3(BS),
+                             want, s, state, pos, ops, nops, coef, ncoef, srcs, (uint32_t)tiles);
+        else
+          hipLaunchKernelGGL((tile_phase_kernel<BS, LB, false>), dim3((unsigned)grid), dim3(BS),
+                             want, s, state, pos, ops, nops, coef, ncoef, srcs, (uint32_t)tiles);
+        return qfx::check_launch("tile_phase_kernel");
+      }
+    }
+  }
   if constexpr (!WIDE && !MF && BS <= kRphaseMaxBlock) {
     // the caller checked T == LB + 4 for these
     if (reg_in) {
@@ -1377,8 +1509,16 @@ int qfx_tile_prepare_ops(qfx_tile_op* ops, int nops) {
 int qfx_tile_check_ops(int T, int block, int flags, const qfx_tile_op* ops, int nops,
                        int ncoef, const int* srcs, int nsrcs) {
   if (flags & ~(QFX_TILE_WIDE | QFX_TILE_PERSISTENT | QFX_TILE_MFMA | QFX_TILE_REG_IO |
-                QFX_TILE_REG_IN))
+                QFX_TILE_REG_IN | QFX_TILE_PHASES))
     return qfx::set_error(QFX_EINVAL, "qfx_tile_check_ops: unknown flags");
+  if (flags & QFX_TILE_PHASES) {
+    bool good = (flags & QFX_TILE_REG_IN) && nops >= 2 && ops;
+    for (int i = 0; good && i < nops; ++i) good = ops[i].kind == OP_RPHASE;
+    if (!good)
+      return qfx::set_error(QFX_EINVAL,
+                            "qfx_tile_check_ops: QFX_TILE_PHASES needs QFX_TILE_REG_IN and at "
+                            "least two ops, all register phases");
+  }
   if (flags & QFX_TILE_REG_IN) {
     if ((flags & (QFX_TILE_WIDE | QFX_TILE_MFMA)) || block > kRphaseMaxBlock ||
         (1 << T) != block * kRegs || nops < 1 || !ops || ops[0].kind != OP_RPHASE)
@@ -1602,9 +1742,13 @@ int qfx_tile_pass(void* stream, void* state, int n, int tile_bits, const int* ti
   const bool mf = (flags & QFX_TILE_MFMA) != 0;
   const bool reg_io = (flags & QFX_TILE_REG_IO) != 0;
   const bool reg_in = (flags & QFX_TILE_REG_IN) != 0;
+  const bool phases = (flags & QFX_TILE_PHASES) != 0;
   if (flags & ~(QFX_TILE_WIDE | QFX_TILE_PERSISTENT | QFX_TILE_MFMA | QFX_TILE_REG_IO |
-                QFX_TILE_REG_IN))
+                QFX_TILE_REG_IN | QFX_TILE_PHASES))
     return qfx::set_error(QFX_EINVAL, "qfx_tile_pass: unknown flags");
+  if (phases && (!reg_in || nops < 2))
+    return qfx::set_error(QFX_EINVAL,
+                          "qfx_tile_pass: QFX_TILE_PHASES needs QFX_TILE_REG_IN and two phases");
   if (reg_in && (wide || mf || block > kRphaseMaxBlock || nops < 1 ||
                  (1 << tile_bits) != block * kRegs))
     return qfx::set_error(QFX_EINVAL,
@@ -1637,7 +1781,7 @@ int qfx_tile_pass(void* stream, void* state, int n, int tile_bits, const int* ti
   auto* c = static_cast<const v2d*>(coef);
   auto* sr = static_cast<const int*>(srcs);
 #define QFX_PASS(BS, LB, W, M) \
-  launch_pass<BS, LB, W, M>(s, st, n, tile_bits, pos, o, nops, c, ncoef, sr, pers, reg_io, reg_in)
+  launch_pass<BS, LB, W, M>(s, st, n, tile_bits, pos, o, nops, c, ncoef, sr, pers, reg_io, reg_in, phases)
   switch (block) {
     case 64:
       if (mf) return wide ? QFX_PASS(64, 6, true, true) : QFX_PASS(64, 6, false, true);

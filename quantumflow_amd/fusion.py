@@ -56,6 +56,7 @@ TILE_PERSISTENT = 2
 TILE_MFMA = 4
 TILE_REG_IO = 8
 TILE_REG_IN = 16
+TILE_PHASES = 32
 MFMA_MIN_BITS = 3
 
 
@@ -1686,6 +1687,8 @@ class HostPlan:
                 fl &= ~TILE_REG_IO
             if fl & TILE_REG_IN and (a > 0 or ops[a].kind != OP_RPHASE):
                 fl &= ~TILE_REG_IN
+            if fl & TILE_REG_IN and b - a > 1 and all(o.kind == OP_RPHASE for o in ops[a:b]):
+                fl |= TILE_PHASES
             self.passes.append(('tile', (k, start + a, b - a, block, fl, bounds[a],
                                          bounds[b] - bounds[a], b == len(ops))))
             a = b

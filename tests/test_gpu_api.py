@@ -222,3 +222,32 @@ def test_w16_kat(qf):
             gates.append(qf.STDGATES[g[0]](*g[1], *g[2]))
     ket = qf.Circuit(gates).run(qf.zero_state(16))
     assert qf.states_close(ket, qf.w_state(16))
+
+
+@pytest.mark.parametrize("n,seed,most", [(22, 1, 464), (23, 1, 644)])
+def test_register_phase_passes_three_to_a_cu(qf, n, seed, most):
+    """Passes of register phases alone in the kernel without prefetch, with
+    both ends (stores from registers and in lane order) and both sizes of its
+    coefficients (up to 512, and more), against the prefetching kernel on the
+    same plan: the same operations in the same order, so the same bits.  At 22
+    qubits the tiles fill its grid once and a third."""
+    import torch
+    from quantumflow_amd import fusion
+    rng = np.random.default_rng(seed)
+    gates = []
+    for _ in range(8 * n):
+        w = 12 if rng.random() < 0.8 else n
+        a, b = rng.choice(w, 2, replace=False).tolist()
+        gates.append([qf.RX(rng.uniform(0, 6), a), qf.H(b), qf.CPHASE(rng.uniform(0, 6), a, b),
+                      qf.CNOT(a, b), qf.TY(rng.uniform(), b), qf.SWAP(a, b),
+                      qf.CPHASE(rng.uniform(0, 6), b, a)][rng.integers(0, 7)])
+    plan = fusion.TilePlan(gates, tuple(range(n)), tile_bits=12, low_bits=3, block=256,
+                           mode='reg')
+    hit = [p for k, p in plan.passes if k == 'tile' and p[4] & fusion.TILE_PHASES]
+    assert {bool(p[4] & fusion.TILE_REG_IO) for p in hit} == {False, True}
+    assert max(p[6] for p in hit) == most
+    psi = torch.randn(2 ** n, dtype=torch.complex128, device='cuda')
+    got = plan.run_inplace(psi.clone())
+    plan.passes = [(k, p[:4] + (p[4] & ~fusion.TILE_PHASES,) + p[5:]) if k == 'tile' else (k, p)
+                   for k, p in plan.passes]
+    assert torch.equal(got, plan.run_inplace(psi.clone()))
