@@ -336,6 +336,13 @@ int qfx_tile_pass(void* stream, void* state, int n, int tile_bits,
                   const void* ops, int nops, const void* coef, int ncoef,
                   const void* srcs, int block, int flags);
 
+/* The same pass from one state to another: `from` is read, `state` written
+ * whole; the two are the same or do not overlap. */
+int qfx_tile_pass_from(void* stream, const void* from, void* state, int n, int tile_bits,
+                       const int* tile_pos /*host*/, const int* dest /*host or NULL*/,
+                       const void* ops, int nops, const void* coef, int ncoef,
+                       const void* srcs, int block, int flags);
+
 /* ---- QAOA MaxCut (quantumflow/qaoa.py) --------------------------------- */
 
 /* Cut table C(z) = sum_e w_e [z_u != z_v] over all 2^n basis states, edges

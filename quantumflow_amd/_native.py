@@ -99,6 +99,7 @@ SIGNATURES = {
     'qfx_tile_prepare_ops': (_i, [_vp, _i]),
     'qfx_tile_check_ops': (_i, [_i, _i, _i, _vp, _i, _i, _ip, _i]),
     'qfx_tile_pass': (_i, [_vp, _vp, _i, _i, _ip, _ip, _vp, _i, _vp, _i, _vp, _i, _i]),
+    'qfx_tile_pass_from': (_i, [_vp, _vp, _vp, _i, _i, _ip, _ip, _vp, _i, _vp, _i, _vp, _i, _i]),
 }
 
 _lib = None

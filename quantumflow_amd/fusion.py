@@ -1759,12 +1759,15 @@ class TilePlan(HostPlan):
                              _native.int_array(p[1][7]) if p[1][7] is not None else None)
                             if p[0] == 'tile' else None for p in self.passes]
 
-    def run_inplace(self, work, prof=None):
-        """Run every pass in place on the flat complex128 device state."""
+    def run_inplace(self, work, prof=None, source=None):
+        """Run every pass in place on the flat complex128 device state; with
+        ``source`` the first pass, a tile pass, reads that state and writes
+        ``work``."""
         s = bk.stream_handle()
         n = self.n
         lib = _native.load()
         wp = _native.ctypes.c_void_p(work.data_ptr())
+        fp = wp if source is None else _native.ctypes.c_void_p(source.data_ptr())
         base_ops = self._ops.data_ptr()
         coef = self._coef.data_ptr()
         srcs = _native.ctypes.c_void_p(self._srcs.data_ptr())
@@ -1776,11 +1779,12 @@ class TilePlan(HostPlan):
             else:
                 pos, start, nops, block, flags, c_lo, ncoef, _ = payload
                 tok = prof.start('tile_pass') if prof is not None else None
-                rc = lib.qfx_tile_pass(s, wp, n, posarr[1], posarr[0], posarr[2],
-                                       _native.ctypes.c_void_p(base_ops + start * self._opsize),
-                                       nops, _native.ctypes.c_void_p(coef + 16 * c_lo), ncoef,
-                                       srcs, block, flags)
+                rc = lib.qfx_tile_pass_from(
+                    s, fp, wp, n, posarr[1], posarr[0], posarr[2],
+                    _native.ctypes.c_void_p(base_ops + start * self._opsize), nops,
+                    _native.ctypes.c_void_p(coef + 16 * c_lo), ncoef, srcs, block, flags)
                 _native.check(rc, 'qfx_tile_pass')
+                fp = wp
             if tok is not None:
                 prof.stop(tok)
         return work
@@ -1788,8 +1792,14 @@ class TilePlan(HostPlan):
     def run(self, ket: State) -> State:
         if tuple(ket.qubits) != self.qubits:
             raise ValueError('plan was built for qubits %s' % (self.qubits,))
-        work = bk.as_device(ket.tensor).clone()
-        self.run_inplace(work)
+        given = bk.as_device(ket.tensor)
+        # a first tile pass reads the given amplitudes where they are laid out
+        # as a copy of them would be
+        direct = (self.passes and self.passes[0][0] == 'tile' and given.is_contiguous()
+                  and not (given.is_conj() or given.is_neg() or given.requires_grad)
+                  and given.data_ptr() % 16 == 0)
+        work = torch.empty_like(given) if direct else given.clone()
+        self.run_inplace(work, source=given if direct else None)
         return State(work.view([2] * self.n), self.qubits, ket.memory)
 
 

@@ -251,3 +251,32 @@ def test_register_phase_passes_three_to_a_cu(qf, n, seed, most):
     plan.passes = [(k, p[:4] + (p[4] & ~fusion.TILE_PHASES,) + p[5:]) if k == 'tile' else (k, p)
                    for k, p in plan.passes]
     assert torch.equal(got, plan.run_inplace(psi.clone()))
+
+
+@pytest.mark.parametrize("cfg", [
+    dict(tile_bits=12, low_bits=3, block=256, mode='reg'),
+    dict(tile_bits=12, low_bits=3, block=256, mode='reg', reg_in=False),
+    dict(tile_bits=12, low_bits=3, block=256, mode='reg', persistent=False),
+    dict(tile_bits=9, low_bits=3, block=64, mode='lds', fuse_width=4),
+    dict(tile_bits=12, low_bits=3, block=256, mode='mfma'),
+])
+@pytest.mark.parametrize("n", [13, 16, 22])
+def test_first_pass_reads_the_given_state(qf, n, cfg):
+    """A plan's run leaves the state it was given as it was and returns the bits
+    of the same plan run in place on a copy, for every kernel a first pass may
+    take, with SWAPs folded into its store."""
+    import torch
+    from quantumflow_amd import fusion
+    rng = np.random.default_rng(n)
+    gates = []
+    for _ in range(4 * n):
+        a, b = rng.choice(n, 2, replace=False).tolist()
+        gates.append([qf.RX(rng.uniform(0, 6), a), qf.H(b), qf.CNOT(a, b), qf.SWAP(a, b),
+                      qf.CPHASE(rng.uniform(0, 6), a, b)][rng.integers(0, 5)])
+    plan = fusion.TilePlan(gates, tuple(range(n)), **cfg)
+    psi = torch.randn(2 ** n, dtype=torch.complex128, device='cuda')
+    before = psi.clone()
+    want = plan.run_inplace(before.clone())
+    got = plan.run(qf.State(psi.view([2] * n), range(n)))
+    assert torch.equal(got.tensor.reshape(-1), want)
+    assert torch.equal(psi, before)
