@@ -1068,7 +1068,7 @@ int qfx_qaoa_check(const qfx_qaoa_inst* insts, int ninst, const qfx_qaoa_pass* p
                    int npasses, const qfx_qaoa_item* items, const int* kstart, int nk, int width,
                    int64_t psi_pool_len, int64_t lam_pool_len, int64_t cnt_pool_len,
                    int64_t val_pool_len, int64_t npartial, int mode, int tile_bits) {
-  if (tile_bits < 0 || tile_bits > kMaxT)
+  if (tile_bits < 0 || tile_bits > (mode == QFX_QAOA_BACKWARD ? kMaxT - 1 : kMaxT))
     return qfx::set_error(QFX_ERANGE, "qfx_qaoa_check: tile_bits out of range");
   const int tmax = tile_bits ? tile_bits : kMaxT;
   for (int i = 0; i < ninst; ++i) {
@@ -1167,14 +1167,14 @@ int qfx_qaoa_run(void* stream, const qfx_qaoa_args* args) {
     return qfx::set_error(QFX_EINVAL, "qfx_qaoa_run: backward needs lam_pool");
   if (a.width < 1 || a.width > kAccum || a.ninst < 1 || a.nk < 1)
     return qfx::set_error(QFX_ERANGE, "qfx_qaoa_run: sizes out of range");
-  if (a.tile_bits < 0 || a.tile_bits > kMaxT)
+  if (a.tile_bits < 0 || a.tile_bits > (a.mode == QFX_QAOA_BACKWARD ? kMaxT - 1 : kMaxT))
     return qfx::set_error(QFX_ERANGE, "qfx_qaoa_run: tile_bits out of range");
   if (a.block != 256 && a.block != 512 && a.block != 1024)
     return qfx::set_error(QFX_EINVAL, "qfx_qaoa_run: block must be 256, 512 or 1024");
   hipStream_t s = qfx::as_stream(stream);
   // programs without cut values hold no weighted instance
   const bool flow = a.tables && a.table_off && a.item_need, weighted = a.val_pool;
-  const bool wide = a.tile_bits == 0 || a.tile_bits > 12;
+  const bool wide = a.tile_bits == 0;
   if (a.mode == QFX_QAOA_BACKWARD && wide)
     return !flow      ? launch_qaoa<true, false, true, true>(s, a)
            : weighted ? launch_qaoa<true, true, true, true>(s, a)

@@ -411,6 +411,9 @@ class QAOABatch:
         self.nitems = len(items)
         psi_len = max(psi_len, single_max)
         lam_len = max(lam_len, single_max)
+        # 13-bit tiles backward go by the engine's default
+        widest = max(ps.T for ps in pass_list)
+        tile_bits = widest if widest <= T_max else 0
         # host-side validation of the whole program
         passes_arr = (QaoaPass * len(pass_list))(*pass_list)
         items_arr = (QaoaItem * len(items))(*items)
@@ -421,7 +424,7 @@ class QAOABatch:
                                          lam_len if mode == MODE_BACKWARD else 0,
                                          max(cnt_len, 1) if cnt_len else 0,
                                          max(val_len, 1) if val_len else 0, nslots, mode,
-                                         max(ps.T for ps in pass_list)),
+                                         tile_bits),
                       'qfx_qaoa_check')
 
         def up(arr):
@@ -473,7 +476,7 @@ class QAOABatch:
             self.sync.data_ptr()
         a.ninst, a.nk, a.width, a.mode, a.block = ninst, self.nk, self.width, mode, block
         a.max_items_per_k = max(kstart[k + 1] - kstart[k] for k in range(self.nk))
-        a.tile_bits = max(ps.T for ps in pass_list)
+        a.tile_bits = tile_bits
         self._need = torch.tensor(need, dtype=torch.int32, device=dev)
         if flow:
             a.tables, a.table_off = self._tables.data_ptr(), self._table_off.data_ptr()
