@@ -1398,11 +1398,12 @@ int launch_pass(hipStream_t s, const v2d* from, v2d* state, int n, int T, const 
   const uint64_t tiles = (uint64_t)1 << (n - T);
   int grid = 0;
   int rc = QFX_OK;
-  // Passes of register phases alone, once the tiles fill the larger grid;
-  // fewer run as well two to a CU with the next tile in flight.  The same 40
-  // layers of gates, three / two to a CU: 22 qubits 484 / 562 us, 23 1054 /
-  // 1138, 25 4022 / 4318, 28 35.1 / 37.0 ms.  Only blocks of 256: one of 512
-  // would leave two waves to a SIMD, without the prefetch.
+  // Passes of register phases alone, three workgroups to a CU.  The same 40
+  // layers of gates, three / two to a CU: 28 qubits 35.1 / 37.0 ms, 25 4022 /
+  // 4318 us, 23 1054 / 1138, 22 484 / 562; where a workgroup has one tile,
+  // which the other kernel loads again as its next, 20 231 / 234, 16 123 /
+  // 128, 14 116 / 120.  Only blocks of 256: one of 512 would leave two waves
+  // to a SIMD, without the prefetch.
   if constexpr (!WIDE && !MF && BS == 256) {
     if (phases) {
       // the coefficients in one of two sizes, so that few grids are asked for
@@ -1411,17 +1412,14 @@ int launch_pass(hipStream_t s, const v2d* from, v2d* state, int n, int T, const 
                               : (const void*)tile_phase_kernel<BS, LB, false>;
       rc = kernel_grid(fn, "tile_phase_kernel", BS, want, &grid);
       if (rc) return rc;
-      if (tiles >= (uint64_t)grid) {
-        if (reg_io)
-          hipLaunchKernelGGL((tile_phase_kernel<BS, LB, true>), dim3((unsigned)grid), dim3(BS),
-                             want, s, from, state, pos, ops, nops, coef, ncoef, srcs,
-                             (uint32_t)tiles);
-        else
-          hipLaunchKernelGGL((tile_phase_kernel<BS, LB, false>), dim3((unsigned)grid), dim3(BS),
-                             want, s, from, state, pos, ops, nops, coef, ncoef, srcs,
-                             (uint32_t)tiles);
-        return qfx::check_launch("tile_phase_kernel");
-      }
+      const unsigned g = tiles < (uint64_t)grid ? (unsigned)tiles : (unsigned)grid;
+      if (reg_io)
+        hipLaunchKernelGGL((tile_phase_kernel<BS, LB, true>), dim3(g), dim3(BS), want, s, from,
+                           state, pos, ops, nops, coef, ncoef, srcs, (uint32_t)tiles);
+      else
+        hipLaunchKernelGGL((tile_phase_kernel<BS, LB, false>), dim3(g), dim3(BS), want, s, from,
+                           state, pos, ops, nops, coef, ncoef, srcs, (uint32_t)tiles);
+      return qfx::check_launch("tile_phase_kernel");
     }
   }
   if constexpr (!WIDE && !MF && BS <= kRphaseMaxBlock) {

@@ -224,13 +224,14 @@ def test_w16_kat(qf):
     assert qf.states_close(ket, qf.w_state(16))
 
 
-@pytest.mark.parametrize("n,seed,most", [(22, 1, 464), (23, 1, 644)])
+@pytest.mark.parametrize("n,seed,most", [(20, 1, 300), (22, 1, 464), (23, 1, 644)])
 def test_register_phase_passes_three_to_a_cu(qf, n, seed, most):
     """Passes of register phases alone in the kernel without prefetch, with
     both ends (stores from registers and in lane order) and both sizes of its
     coefficients (up to 512, and more), against the prefetching kernel on the
-    same plan: the same operations in the same order, so the same bits.  At 22
-    qubits the tiles fill its grid once and a third."""
+    same plan: the same operations in the same order, so the same bits.  At 20
+    qubits a workgroup has one tile, at 22 the tiles fill the grid once and a
+    third."""
     import torch
     from quantumflow_amd import fusion
     rng = np.random.default_rng(seed)
