@@ -58,10 +58,11 @@ def _runs(elements, item):
             yield None, elem
 
 
-def _bits_of(qubits):
-    """Index bit of each qubit label of a state."""
-    n = len(qubits)
-    return {q: n - 1 - i for i, q in enumerate(qubits)}
+def _bits_of(qubits, axes):
+    """Index bit of each qubit label's first axis in a tensor of ``axes`` axes:
+    a state has one axis per label, a density or a gate its row axes, then its
+    column axes."""
+    return {q: axes - 1 - i for i, q in enumerate(qubits)}
 
 
 def _lookup(bit_of, qubits):
@@ -138,11 +139,11 @@ class Circuit(Operation):
             # each element's kernel gates act on its qubits' row axes, then
             # (or also) on their column axes
             n = rho.qubit_nb
-            bit_of = _bits_of(rho.qubits)
+            bit_of = _bits_of(rho.qubits, 2 * n)
             kinds, bits = [], []
             for e, gates in run:
-                cols = _lookup(bit_of, e.qubits)
-                rows = [b + n for b in cols]
+                rows = _lookup(bit_of, e.qubits)
+                cols = [b - n for b in rows]
                 for kind, where in gates:
                     kinds.append(kind)
                     bits += rows + cols if where == 'both' else \
@@ -195,7 +196,8 @@ class Circuit(Operation):
             if run is None:
                 ket = elem.run(ket)
                 continue
-            bit_of = _bits_of(ket.qubits)
+            # a density's gates act on its row axes, as Gate.run's do
+            bit_of = _bits_of(ket.qubits, bk.rank(ket.tensor))
             bits = [b for gate, _ in run for b in _lookup(bit_of, gate.qubits)]
             tensor = bk.apply_gates(ket.tensor, [kind for _, kind in run], bits)
             ket = State(tensor, ket.qubits, ket.memory)
@@ -214,7 +216,7 @@ class Circuit(Operation):
                 gate = elem.asgate() @ (identity_gate(qubits) if gate is None else gate)
                 continue
             n = len(qubits)
-            bit_of = {q: b + n for q, b in _bits_of(qubits).items()}
+            bit_of = _bits_of(qubits, 2 * n)
             bits = [b for g, _ in run for b in _lookup(bit_of, g.qubits)]
             tensor = bk.identity_tensor(n) if gate is None else gate.tensor
             gate = Gate(tensor=bk.apply_gates(tensor, [kind for _, kind in run], bits),

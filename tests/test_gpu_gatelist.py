@@ -78,6 +78,20 @@ def test_small_circuit_with_measurement_and_nested_circuit(qf):
         qf.Circuit([qf.H(0), qf.X(7)]).run(qf.zero_state(2))
 
 
+@pytest.mark.parametrize("n", [1, 2, 3, 6, 7, 8])
+def test_run_on_a_density_matches_per_gate_path(qf, n):
+    # run multiplies a density's rows alone; 2 to 16 index bits
+    rng = np.random.default_rng(60 + n)
+    circ = qf.Circuit(_rand_gates(qf, n, 25, rng))
+    rho = qf.State(_rand_state(n, rng), range(n)).asdensity()
+    got = circ.run(rho)
+    plain = circ.run(rho, fused=False)
+    assert type(got) is type(plain) and got.qubits == plain.qubits
+    # 25 gates on entries of at most 1, up to 16 terms a sum: gates that share
+    # no qubit may change places
+    assert np.max(np.abs(got.vec.asarray() - plain.vec.asarray())) <= 25 * 16 * 2.0 ** -53
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 5, 6, 7, 8])
 def test_density_circuits_match_element_by_element(qf, n):
     # 2n from 2 to 16 index bits: whole-state tiles, then passes of 12 bits
