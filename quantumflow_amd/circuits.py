@@ -210,7 +210,9 @@ class Circuit(Operation):
         gate = None
 
         def item(elem):
-            return _listed(elem, 'asgate') if type(elem).__matmul__ is Gate.__matmul__ else None
+            if isinstance(elem, Gate) and type(elem).__matmul__ is Gate.__matmul__:
+                return _listed(elem, 'asgate')
+            return None                         # nested circuits among them
         for run, elem in _runs(self.elements, item):
             if run is None:
                 gate = elem.asgate() @ (identity_gate(qubits) if gate is None else gate)

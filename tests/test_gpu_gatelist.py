@@ -130,6 +130,20 @@ def test_composed_gate_matches_products(qf, k):
     assert np.max(np.abs(got.matrix - want.reshape(2 ** k, 2 ** k))) <= 1e-13
 
 
+@pytest.mark.parametrize("n", [2, 5, 8])
+def test_nested_circuits_match_flat_ones(qf, n):
+    rng = np.random.default_rng(90 + n)
+    gates = _rand_gates(qf, n, 12, rng) + [qf.RX(0.1 * q, q) for q in range(n)]
+    flat = qf.Circuit(gates)
+    nested = qf.Circuit([qf.Circuit(gates[:3]), gates[3], qf.Circuit([qf.Circuit(gates[4:6])]),
+                         qf.Circuit(gates[6:9])] + gates[9:])
+    ket = qf.State(_rand_state(n, rng), range(n))
+    assert np.array_equal(nested.run(ket).vec.asarray(), flat.run(ket).vec.asarray())
+    # 20 unitaries of at most 16 terms a row, multiplied in another grouping
+    assert nested.asgate().qubits == flat.asgate().qubits
+    assert np.max(np.abs(nested.asgate().matrix - flat.asgate().matrix)) <= 20 * 16 * 2.0 ** -53
+
+
 def test_records_are_checked(qf):
     from quantumflow_amd import _native, backend as bk
     ket = qf.zero_state(3).tensor
