@@ -362,6 +362,15 @@ class GateKind:
             ph = m[np.arange(dim), self.src]
             self.phase = None if all(z == 1.0 for z in ph.tolist()) else ph
 
+    def __getstate__(self):
+        # the native record holds addresses: a copy makes its own
+        return None, {name: getattr(self, name) for name in self.__slots__ if name != '_record'}
+
+    def __setstate__(self, state):
+        for name, value in state[1].items():
+            setattr(self, name, value)
+        self._record = None
+
     @property
     def listable(self):
         """Whether qfx_apply_gates takes this gate."""

@@ -1,5 +1,7 @@
 """How circuits hand their gates to the gate-list kernel (no GPU: the calls
 that would launch are recorded instead)."""
+import copy
+import pickle
 from types import SimpleNamespace
 
 import numpy as np
@@ -95,3 +97,30 @@ def test_asgate_keeps_the_error_of_operations_without_a_gate(on_host):
         qf.Circuit([qf.X(0), qf.Measure(0)]).asgate()
     with pytest.raises(TypeError):
         qf.Circuit([qf.X(0), qf.Damping(0.1, 0)]).asgate()
+
+
+@pytest.mark.parametrize("gate", [qf.RX(0.3, 0), qf.RZ(0.7, 1), qf.ISWAP(0, 1)])
+def test_gates_are_copied_and_pickled_after_a_run(gate):
+    # what a run leaves with the gate: its class and native record
+    rec = gate.kind.record()
+    assert gate.kind.record() is rec
+    copies = [copy.copy(gate.kind), copy.deepcopy(gate).kind]
+    copies += [pickle.loads(pickle.dumps(gate, protocol)).kind for protocol in (2, 3, 4, 5)]
+    for kind in copies:
+        assert (kind.kind, kind.k) == (gate.kind.kind, gate.kind.k)
+        for name in ('matrix', 'diag', 'src', 'phase'):
+            a, b = getattr(kind, name), getattr(gate.kind, name)
+            assert (a is None and b is None) or np.array_equal(a, b)
+        # a record of its own, with the same contents
+        own = kind.record()
+        assert own[0] != rec[0]
+        assert (own[1].kind, own[1].k) == (rec[1].kind, rec[1].k)
+        for a, b in zip(own[2:], rec[2:]):
+            assert (a is None and b is None) or np.array_equal(a, b)
+
+
+def test_class_pickled_without_a_record_slot_loads():
+    kind = qf.ISWAP(0, 1).kind
+    old = type(kind).__new__(type(kind))
+    old.__setstate__((None, {n: getattr(kind, n) for n in kind.__slots__ if n != '_record'}))
+    assert old.record()[1].k == 2

@@ -144,6 +144,20 @@ def test_nested_circuits_match_flat_ones(qf, n):
     assert np.max(np.abs(nested.asgate().matrix - flat.asgate().matrix)) <= 20 * 16 * 2.0 ** -53
 
 
+def test_circuits_are_copied_and_pickled_after_a_run(qf):
+    import copy
+    import pickle
+    rng = np.random.default_rng(8)
+    circ = qf.Circuit(_rand_gates(qf, 4, 12, rng))
+    ket = qf.State(_rand_state(4, rng), range(4))
+    want = circ.run(ket).vec.asarray()
+    circ.asgate()
+    for g in circ.elements:
+        g.tensor                                # the device copy goes along
+    for other in (copy.deepcopy(circ), pickle.loads(pickle.dumps(circ))):
+        assert np.array_equal(other.run(ket).vec.asarray(), want)
+
+
 def test_records_are_checked(qf):
     from quantumflow_amd import _native, backend as bk
     ket = qf.zero_state(3).tensor
