@@ -145,9 +145,9 @@ def instance_groups(state_bytes, limit):
     """Instances in the order their items are listed, by the state they keep
     and as many to a group as keep at most `limit` bytes (at least one)."""
     order = sorted(range(len(state_bytes)), key=lambda i: state_bytes[i])
-    groups, held = [], math.inf
+    groups, held = [], 0
     for i in order:
-        if held + state_bytes[i] > limit:
+        if not groups or held + state_bytes[i] > limit:
             groups.append([])
             held = 0
         groups[-1].append(i)

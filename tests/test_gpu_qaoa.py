@@ -417,3 +417,39 @@ def test_wide_backward_tiles(E, monkeypatch):
         res.append((val.cpu().numpy().copy(), grad.cpu().numpy().copy()))
     assert np.max(np.abs(res[0][0] - res[1][0])) <= 2e-10
     assert np.max(np.abs(res[0][1] - res[1][1])) <= 2e-10
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_batches_that_keep_too_much_for_item_waits(E, mode, monkeypatch):
+    """A batch with an instance past FLOW_KEPT is built for grid barriers and
+    gives the same values and gradients: within 2 * 6e-11, twice the bound
+    that either way keeps against 64 bits (14 qubits, 4 layers)."""
+    rng = np.random.default_rng(31 + mode)
+    graphs = [er(n, 0.5, 5 * n) for n in (3, 9, 13, 14)]
+    beta, gamma = rng.uniform(-4, 4, size=(2, len(graphs), 4))
+    res = []
+    for kept in (E.FLOW_KEPT, 0):
+        monkeypatch.setattr(E, 'FLOW_KEPT', kept)
+        b = E.QAOABatch(graphs, 4, mode=mode)
+        assert bool(b._args.tables) == bool(b._args.item_need) == (kept > 0)
+        val, grad = b.evaluate(beta, gamma)
+        b.check()
+        res.append([x.cpu().numpy().copy() for x in (val, grad) if x is not None])
+    for a, b in zip(*res):
+        assert np.max(np.abs(a - b)) <= 1.2e-10
+
+
+def test_state_past_item_waits(E):
+    """28 qubits whole keep 2^28 amplitudes (grid barriers), mirrored 2^27
+    (item waits).  An amplitude gathers about 3 roundings of 2^-53 a qubit and
+    layer: either value within 3 * 28 * 2^-53 |E|^2 < 2e-11 (42 edges)."""
+    g = nx.random_regular_graph(3, 28, seed=1)
+    vals = []
+    for mirror in (False, True):
+        b = E.QAOABatch([g], 1, mode=E.MODE_FORWARD, mirror=mirror)
+        assert bool(b._args.tables) == mirror
+        vals.append(b.evaluate([[0.6]], [[0.9]])[0][0].item())
+        b.check()
+        del b
+    assert abs(vals[0] - vals[1]) <= 4e-11
+    assert 0 < vals[0] < 42

@@ -306,3 +306,20 @@ def test_mirror_program_on_tiles_matches_oracle(n, T, p):
     ref = O.qaoa_expectation(n, edges, beta, gamma)
     assert E.use_mirror(n, T)
     assert abs(_emulate_mirror_tiles(n, edges, beta, gamma, T) - ref) < 1e-12
+
+
+@pytest.mark.parametrize("limit", [1, 100, 10 ** 6, float('inf')])
+def test_instance_groups_hold_every_instance_once(limit):
+    """By ascending state, none above the limit unless it is one instance's;
+    without a limit (instances of 2^28 kept amplitudes and more) all are one
+    group."""
+    state = [0, 64, 0, 32, 2 ** 32, 64]
+    groups = E.instance_groups(state, limit)
+    listed = [i for g in groups for i in g]
+    assert sorted(listed) == list(range(len(state)))
+    assert [state[i] for i in listed] == sorted(state)
+    assert all(len(g) == 1 or sum(state[i] for i in g) <= limit for g in groups)
+    if limit == float('inf'):
+        assert len(groups) == 1
+    assert E.instance_groups([], limit) == []
+    assert E.instance_groups([2 ** 32], limit) == [[0]]
