@@ -176,8 +176,12 @@ int qfx_plus_state(void* stream, void* psi, int n);
  * drawn with probability |psi_i|^2 / sum_j |psi_j|^2, from a SplitMix64
  * stream keyed by (seed, t); reproducible for equal (psi, seed).  Indices of
  * zero probability are never drawn.  Index bit n-1-a is qubit axis a. */
-/* Bytes of device workspace qfx_sample needs for n qubits (0 if n invalid). */
+/* Bytes of device workspace qfx_sample needs for n qubits and any number of
+ * draws (0 if n invalid); from n = 11 to 30 about 1/32 of the state. */
 int64_t qfx_sample_workspace_bytes(int n);
+/* The same for a call of `trials` draws: few draws (below 1024, or 2^(n-15)
+ * above 25 qubits) need 1/1024 of the state. */
+int64_t qfx_sample_workspace_bytes_for(int n, int64_t trials);
 int qfx_sample(void* stream, int64_t* out, const void* psi, int n,
                int64_t trials, uint64_t seed, void* workspace);
 /* counts[idx[i]] += 1 for i < m (counts: 2^n int64, zeroed by the caller;

@@ -73,6 +73,7 @@ SIGNATURES = {
     'qfx_zero_state': (_i, [_vp, _vp, _i]),
     'qfx_plus_state': (_i, [_vp, _vp, _i]),
     'qfx_sample_workspace_bytes': (_i64, [_i]),
+    'qfx_sample_workspace_bytes_for': (_i64, [_i, _i64]),
     'qfx_sample': (_i, [_vp, _vp, _vp, _i, _i64, ctypes.c_uint64, _vp]),
     'qfx_histogram': (_i, [_vp, _vp, _vp, _i64, _i]),
     'qfx_density_outer': (_i, [_vp, _vp, _vp, _i]),

@@ -621,9 +621,9 @@ def sample_indices(tensor: BKTensor, trials: int, seed: int) -> BKTensor:
     out = torch.empty(trials, dtype=torch.int64, device=a.device)
     if trials == 0:
         return out
-    # the allocator's, not the kept scratch: it holds 1/32 of the state
-    ws = torch.empty(_native.load().qfx_sample_workspace_bytes(n), dtype=torch.uint8,
-                     device=a.device)
+    # the allocator's, not the kept scratch: for many draws 1/32 of the state
+    ws = torch.empty(_native.load().qfx_sample_workspace_bytes_for(n, trials),
+                     dtype=torch.uint8, device=a.device)
     _native.call('qfx_sample', stream_handle(), _ptr(out), _ptr(a), n, trials,
                  int(seed) & (2 ** 64 - 1), _ptr(ws))
     return out

@@ -354,15 +354,23 @@ constexpr int kMaxTableQubits = 30;
 // draws.
 int64_t table_trials(int n) { return n > 25 ? (int64_t)1 << (n - 15) : 1024; }
 
+bool uses_table(int n, int64_t trials) {
+  return n <= kMaxTableQubits && trials >= table_trials(n);
+}
+
 }  // namespace
 
 extern "C" {
 
-int64_t qfx_sample_workspace_bytes(int n) {
+int64_t qfx_sample_workspace_bytes_for(int n, int64_t trials) {
   if (n < 1 || n > QFX_MAX_QUBITS) return 0;
   const uint64_t nchunks = (uint64_t)1 << (n - chunk_bits(n));
-  const uint64_t table = n <= kMaxTableQubits ? nchunks * kSegs : 0;
+  const uint64_t table = uses_table(n, trials) ? nchunks * kSegs : 0;
   return (int64_t)(sizeof(double) * (2 * nchunks + 1 + scan_segments(nchunks) + table));
+}
+
+int64_t qfx_sample_workspace_bytes(int n) {
+  return qfx_sample_workspace_bytes_for(n, INT64_MAX);
 }
 
 int qfx_sample(void* stream, int64_t* out, const void* psi, int n, int64_t trials,
@@ -379,7 +387,7 @@ int qfx_sample(void* stream, int64_t* out, const void* psi, int n, int64_t trial
   double* pre = sums + nchunks;
   double* seg = pre + nchunks + 1;
   double* tab = seg + nseg;
-  const bool table = n <= kMaxTableQubits && trials >= table_trials(n);
+  const bool table = uses_table(n, trials);
   auto* st = static_cast<const double2*>(psi);
   const dim3 sgrid((unsigned)((nchunks + kSumWaves - 1) / kSumWaves)), sblock(64 * kSumWaves);
   if (table)

@@ -58,3 +58,19 @@ def test_workspace_size_formula():
     lib = _native.load()
     assert lib.qfx_reduce_workspace_bytes(1 << 28) >= (1 << 12) * 17 * 8
     assert lib.qfx_reduce_workspace_bytes(4) >= 1024 * 16
+
+
+@pytest.mark.parametrize("n", [1, 10, 11, 20, 25, 26, 28, 30, 31, 34])
+def test_sample_workspace_by_draws(n):
+    lib = _native.load()
+    chunks = 2 ** max(n - 10, 0)
+    few = 8 * (2 * chunks + 1 + (chunks + 1023) // 1024)
+    many = few + (8 * 64 * chunks if n <= 30 else 0)
+    first = 2 ** (n - 15) if n > 25 else 1024
+    for trials in (-1, 0, 1, first - 1):
+        assert lib.qfx_sample_workspace_bytes_for(n, trials) == few
+    for trials in (first, 2 ** 40):
+        assert lib.qfx_sample_workspace_bytes_for(n, trials) == many
+    assert lib.qfx_sample_workspace_bytes(n) == many
+    assert lib.qfx_sample_workspace_bytes_for(0, 1) == 0
+    assert lib.qfx_sample_workspace_bytes_for(35, 1) == 0

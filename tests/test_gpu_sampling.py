@@ -289,3 +289,31 @@ def test_fused_segments_around_measure_and_reset(qf):
         err = np.max(np.abs(a.vec.asarray() - b.vec.asarray()))
         print(f"seed {seed}: memory {dict(a.memory)} max |d amp| {err:.2e}")
         assert err < 1e-12
+
+
+@pytest.mark.parametrize("n", [6, 11, 21, 26])
+@pytest.mark.parametrize("many", [False, True])
+def test_draws_stay_in_their_workspace(qf, n, many):
+    # the numbers of draws on both sides of the segment table: nothing past the
+    # bytes asked for is written, and few draws take no table
+    import torch
+    from quantumflow_amd import _native, backend as bk
+    ket = qf.zero_state(n).tensor.reshape(-1).clone()
+    ket[1:] = 2.0 ** -n
+    first = 2 ** (n - 15) if n > 25 else 1024
+    trials = first if many else first - 1
+    lib = _native.load()
+    size = lib.qfx_sample_workspace_bytes_for(n, trials)
+    ws = torch.full((size + 4096,), 77, dtype=torch.uint8, device='cuda')
+    out = torch.empty(trials, dtype=torch.int64, device='cuda')
+    ptr = [_native.ctypes.c_void_p(t.data_ptr()) for t in (out, ket, ws)]
+    _native.call('qfx_sample', bk.stream_handle(), ptr[0], ptr[1], n, trials, 5, ptr[2])
+    assert bool((ws[size:] == 77).all())
+    assert torch.equal(out, bk.sample_indices(ket, trials, 5))
+    if not many:
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        bk.sample_indices(ket, 1, 5)
+        torch.cuda.synchronize()
+        assert torch.cuda.max_memory_allocated() - before <= 2 ** (n + 4) // 512 + 4096
