@@ -14,6 +14,7 @@
 //             the tile with the kLowBits lowest bits (contiguous runs); a gate
 //             may pass one that is left behind if they share no bit.  A pass
 //             of one gate runs on the per-gate kernels.
+#include <algorithm>
 #include <cstddef>
 #include <cstring>
 #include <string>
@@ -407,6 +408,7 @@ struct Item {
   const qfx_gate* g;
   const int* bits;
   uint64_t mask;
+  int units;                            // as an op of its own (item_units)
 };
 
 bool is_one(const qfx_c128& z) { return z.re == 1.0 && z.im == 0.0; }
@@ -617,7 +619,7 @@ int qfx_apply_gates(void* stream, void* out, const void* in, int n, int ngates,
         seen |= 1u << g->src[r];
       }
     }
-    items[i] = Item{g, bits, 0};
+    items[i] = Item{g, bits, 0, item_units(*g)};
     for (int j = 0; j < g->k; ++j) items[i].mask |= (uint64_t)1 << bits[j];
     bits += g->k;
   }
@@ -645,7 +647,7 @@ int qfx_apply_gates(void* stream, void* out, const void* in, int n, int ngates,
   if (n <= kWholeBits) {
     set_tile(((uint64_t)1 << n) - 1);
     for (const Item& it : items) {
-      if (!p.fits(item_units(*it.g))) {
+      if (!p.fits(it.units)) {
         const int rc = flush();
         if (rc) return rc;
       }
@@ -653,31 +655,45 @@ int qfx_apply_gates(void* stream, void* out, const void* in, int n, int ngates,
     }
     return flush();
   }
-  const uint64_t low = ((uint64_t)1 << kLowBits) - 1;
-  std::vector<int> pending(items.size()), left, take;
-  for (size_t i = 0; i < items.size(); ++i) pending[i] = (int)i;
-  while (!pending.empty()) {
+  // A pass looks at the gates that earlier ones passed over, left[head ..],
+  // then at those from `next` on, until none can join it any more: so far and
+  // no further, or a list of many passes would cost the square of its length.
+  const uint64_t low = ((uint64_t)1 << kLowBits) - 1, all = ((uint64_t)1 << n) - 1;
+  std::vector<int> left, over, take;
+  size_t head = 0, next = 0;
+  while (head < left.size() || next < items.size()) {
     uint64_t tile = low, blocked = 0;
     int units = 0;
-    bool full = false;
-    left.clear();
+    over.clear();
     take.clear();
-    for (int i : pending) {
+    // takes gate i or passes over it; false once no later gate can be taken
+    auto offer = [&](int i) {
       const Item& it = items[i];
-      const int u = item_units(*it.g);
-      if (!full && !(it.mask & blocked) && __builtin_popcountll(tile | it.mask) <= kTileBits) {
-        if (units + u <= kUnits) {
+      if (!(it.mask & blocked) && __builtin_popcountll(tile | it.mask) <= kTileBits) {
+        if (units + it.units <= kUnits) {
           tile |= it.mask;
-          units += u;
+          units += it.units;
           take.push_back(i);
-          continue;
+          return true;
         }
-        full = true;
+        over.push_back(i);
+        return false;
       }
       blocked |= it.mask;
-      left.push_back(i);
+      over.push_back(i);
+      return blocked != all && (__builtin_popcountll(tile) < kTileBits || (tile & ~blocked) != 0);
+    };
+    bool open = true;
+    size_t at = head;
+    while (open && at < left.size()) open = offer(left[at++]);
+    if (open) {
+      while (open && next < items.size()) open = offer((int)next++);
+      left.swap(over);
+      head = 0;
+    } else {
+      head = at - over.size();
+      std::copy(over.begin(), over.end(), left.begin() + (ptrdiff_t)head);
     }
-    pending.swap(left);
     if (take.size() == 1) {
       const int rc = run_single(stream, out, src, n, items[take[0]]);
       if (rc) return rc;

@@ -116,6 +116,33 @@ def test_density_circuits_match_element_by_element(qf, n):
     assert abs(complex(got.trace().item()) - 1) <= 1e-12
 
 
+def test_long_lists_take_linear_time(qf):
+    # 16 index bits, where a list is many passes: a gate of 128000 costs what
+    # one of 4000 does (about 1 us; 3.3 us when every pass read the whole list)
+    import time
+    import torch
+    from quantumflow_amd import backend as bk
+    rng = np.random.default_rng(2)
+    state = bk.zero_state_tensor(16)
+    rx, cnot = qf.RX(0.4, 0).kind, qf.CNOT(0, 1).kind
+
+    def per_gate(count):
+        kinds, bits = [], []
+        for i in range(count):
+            kinds.append(cnot if i % 3 == 2 else rx)
+            bits += [int(b) for b in rng.permutation(16)[:kinds[-1].k]]
+        best = np.inf
+        for _ in range(3):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            bk.apply_gates(state, kinds, bits)
+            torch.cuda.synchronize()
+            best = min(best, time.perf_counter() - t0)
+        return best / count
+    short = per_gate(4000)
+    assert per_gate(128000) <= 2 * short
+
+
 @pytest.mark.parametrize("k", [1, 3, 6, 7, 8])
 def test_composed_gate_matches_products(qf, k):
     rng = np.random.default_rng(70 + k)
