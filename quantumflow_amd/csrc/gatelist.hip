@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cstddef>
 #include <cstring>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -590,12 +591,8 @@ int run_single(void* stream, void* out, const void* in, int n, const Item& it) {
                    : qfx_apply_monomial(stream, out, in, n, g.k, it.bits, g.src, g.coef);
 }
 
-}  // namespace
-
-extern "C" {
-
-int qfx_apply_gates(void* stream, void* out, const void* in, int n, int ngates,
-                    const qfx_gate* const* gates, const int* bits) {
+int apply_gates(void* stream, void* out, const void* in, int n, int ngates,
+                const qfx_gate* const* gates, const int* bits) {
   const char* fn = "qfx_apply_gates";
   if (!out || !in || !gates || !bits)
     return qfx::set_error(QFX_EINVAL, std::string(fn) + ": null pointer");
@@ -707,6 +704,19 @@ int qfx_apply_gates(void* stream, void* out, const void* in, int n, int ngates,
     if (rc) return rc;
   }
   return QFX_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int qfx_apply_gates(void* stream, void* out, const void* in, int n, int ngates,
+                    const qfx_gate* const* gates, const int* bits) {
+  try {
+    return apply_gates(stream, out, in, n, ngates, gates, bits);
+  } catch (const std::bad_alloc&) {      // the list's own vectors
+    return qfx::set_error(QFX_EHIP, "qfx_apply_gates: out of host memory");
+  }
 }
 
 }  // extern "C"

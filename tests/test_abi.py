@@ -4,6 +4,7 @@ error codes map onto the reference's exception types.  No kernel runs."""
 import ctypes
 import os
 import subprocess
+import sys
 
 import pytest
 
@@ -74,3 +75,29 @@ def test_sample_workspace_by_draws(n):
     assert lib.qfx_sample_workspace_bytes(n) == many
     assert lib.qfx_sample_workspace_bytes_for(0, 1) == 0
     assert lib.qfx_sample_workspace_bytes_for(35, 1) == 0
+
+
+def test_gate_list_without_memory_for_it_is_an_error():
+    """Host memory that runs out in qfx_apply_gates comes back as an error
+    code, not as an exception out of a C function."""
+    code = '''
+import ctypes, resource
+from quantumflow_amd import _native
+lib = _native.load()
+z = (ctypes.c_double * 8)(0, 0, 1, 0, 1, 0, 0, 0)
+gate = _native.QfxGate(0, 1, ctypes.addressof(z), None)
+count = 1 << 23
+gates = (ctypes.c_void_p * count)(*([ctypes.addressof(gate)] * count))
+bits = (ctypes.c_int * count)()
+pages = int(open('/proc/self/statm').read().split()[0])
+limit = pages * resource.getpagesize() + (16 << 20)
+resource.setrlimit(resource.RLIMIT_AS, (limit, limit))
+p = ctypes.c_void_p(16)
+rc = lib.qfx_apply_gates(None, p, p, 14, count, gates, bits)
+assert rc == _native.QFX_EHIP, rc
+assert 'memory' in _native.last_error(), _native.last_error()
+print('refused')
+'''
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, '-c', code], cwd=root, capture_output=True, text=True)
+    assert run.returncode == 0 and 'refused' in run.stdout, (run.returncode, run.stderr)
