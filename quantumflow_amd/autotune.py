@@ -160,14 +160,17 @@ def store_qaoa(mode, cfg, ms):
 def tune_qaoa(graphs, p, mode, reps=3, candidates=None, store=True, verbose=False):
     """Time the batched engine on these instances for each candidate
     {tile_bits, block} (one HIP-graph replay per repetition) and cache the
-    fastest for the mode.  Returns (best config, {config tuple: ms})."""
+    fastest for the mode.  The kernel runs 512 lanes whatever the block, so the
+    default candidates differ in tile width alone (104 values of 10 to 22
+    qubits with blocks of 256, 512 and 1024: 881, 882 and 870 us, where one
+    block's runs differ by 100; gradients the same to the bit).  Returns (best
+    config, {config tuple: ms})."""
     import numpy as np
     import torch
     from . import qaoa_engine as E
     if candidates is None:
         tmax = 12 if mode == E.MODE_BACKWARD else 13
-        candidates = [dict(tile_bits=t, block=b)
-                      for t, b in itertools.product((tmax, tmax - 1), (256, 512))]
+        candidates = [dict(tile_bits=t, block=512) for t in (tmax, tmax - 1)]
     rng = np.random.default_rng(0)
     beta = rng.uniform(0, np.pi / 2, (len(graphs), p))
     gamma = rng.uniform(0, np.pi, (len(graphs), p))

@@ -53,3 +53,16 @@ def test_tune_qaoa_picks_fastest_and_batches_use_it(cache):
             for c in cands]
     for a, b in zip(outs[0], outs[1]):
         assert np.max(np.abs(a.cpu().numpy() - b.cpu().numpy())) < 1e-11
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", [0, 1])
+def test_tune_qaoa_times_no_program_twice(cache, mode):
+    import networkx as nx
+    from quantumflow_amd import autotune
+    graphs = [nx.cycle_graph(n) for n in (6, 14)]
+    best, results = autotune.tune_qaoa(graphs, 2, mode, reps=1, store=False)
+    widths = [dict(cfg)['tile_bits'] for cfg in results]
+    assert len(widths) > 1 and len(set(widths)) == len(widths)
+    assert best['tile_bits'] in widths and best['block'] == 512
+    assert not cache.exists()
