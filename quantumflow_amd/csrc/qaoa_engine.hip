@@ -34,6 +34,7 @@
 // with lambda, psi carried back by RX(-beta) and the conjugate phases.
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <type_traits>
 
 #include "qfx_common.h"
@@ -985,49 +986,56 @@ __global__ __launch_bounds__(kPrepBlock) void prepare_kernel(
 }
 
 // Persistent grid of one instantiation on one device: every workgroup that
-// fits the device at once (occupancy x CUs for this block size, mode and LDS
-// size), so all of them are resident together and the grid barrier cannot
-// wait on a workgroup that has not started.  Cached per device and LDS size.
-struct GridCache {
+// fits the device at once (occupancy x CUs for this mode), so all of them are
+// resident together and the grid barrier cannot wait on a workgroup that has
+// not started.  Made once per device; other threads wait until it is whole.
+struct Grid {
   int grid = 0;
-  size_t lds = 0;
   uint64_t limit_ticks = 0;
 };
+
+int make_grid(const void* fn, size_t lds, int dev, Grid* to) {
+  int rc = qfx::check_hip(
+      hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+      "hipFuncSetAttribute");
+  if (rc) return rc;
+  int per_cu = 0, cus = 0, rate_khz = 0;
+  rc = qfx::check_hip(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kThreads, lds),
+                      "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+  if (rc) return rc;
+  if (per_cu < 1) return qfx::set_error(QFX_ERANGE, "qfx_qaoa_run: kernel does not fit a CU");
+  rc = qfx::check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev),
+                      "hipDeviceGetAttribute");
+  if (rc) return rc;
+  rc = qfx::check_hip(hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, dev),
+                      "hipDeviceGetAttribute");
+  if (rc) return rc;
+  if (rate_khz <= 0) return qfx::set_error(QFX_EKERNEL, "qfx_qaoa_run: no wall-clock rate");
+  to->grid = per_cu * cus;
+  to->limit_ticks = (uint64_t)rate_khz * 1000u * kBarrierSeconds;
+  return QFX_OK;
+}
 
 template <bool BWD, bool FLOW, bool WTD, bool WIDE>
 int launch_qaoa(hipStream_t s, const qfx_qaoa_args& a) {
   const size_t lds = sizeof(v2d) * kExchange;
-  static GridCache cache[kMaxDevices];
+  static std::mutex mu;
+  static Grid made[kMaxDevices];
   int dev = 0;
   int rc = qfx::check_hip(hipGetDevice(&dev), "hipGetDevice");
   if (rc) return rc;
   if (dev < 0 || dev >= kMaxDevices)
     return qfx::set_error(QFX_ERANGE, "qfx_qaoa_run: device index out of range");
-  GridCache& gc = cache[dev];
-  if (gc.grid == 0 || gc.lds != lds) {
-    rc = qfx::check_hip(hipFuncSetAttribute((const void*)qaoa_kernel<BWD, FLOW, WTD, WIDE>,
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
-                        "hipFuncSetAttribute");
-    if (rc) return rc;
-    int per_cu = 0, cus = 0, rate_khz = 0;
-    rc = qfx::check_hip(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                            &per_cu, (const void*)qaoa_kernel<BWD, FLOW, WTD, WIDE>, kThreads, lds),
-                        "hipOccupancyMaxActiveBlocksPerMultiprocessor");
-    if (rc) return rc;
-    if (per_cu < 1) return qfx::set_error(QFX_ERANGE, "qfx_qaoa_run: kernel does not fit a CU");
-    rc = qfx::check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev),
-                        "hipDeviceGetAttribute");
-    if (rc) return rc;
-    rc = qfx::check_hip(hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, dev),
-                        "hipDeviceGetAttribute");
-    if (rc) return rc;
-    if (rate_khz <= 0) return qfx::set_error(QFX_EKERNEL, "qfx_qaoa_run: no wall-clock rate");
-    gc.grid = per_cu * cus;
-    gc.lds = lds;
-    gc.limit_ticks = (uint64_t)rate_khz * 1000u * kBarrierSeconds;
+  Grid gc;
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (made[dev].grid == 0) {
+      rc = make_grid((const void*)qaoa_kernel<BWD, FLOW, WTD, WIDE>, lds, dev, &made[dev]);
+      if (rc) return rc;
+    }
+    gc = made[dev];
   }
-  const int grid = gc.grid;
-  int g = grid;
+  int g = gc.grid;
   if (a.max_items_per_k > 0 && a.max_items_per_k < g) g = a.max_items_per_k;
   auto* sync = static_cast<unsigned*>(a.sync);
   auto* err = reinterpret_cast<int*>(sync + 1);

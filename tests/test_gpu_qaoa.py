@@ -453,3 +453,35 @@ def test_state_past_item_waits(E):
         del b
     assert abs(vals[0] - vals[1]) <= 4e-11
     assert 0 < vals[0] < 42
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_batches_of_several_threads(E, mode):
+    """Threads that launch at once, each its own batch on its own stream, get
+    the bits of launches one by one.  15 qubits: several passes, so that items
+    wait, but workgroups enough for all of the batches at once."""
+    import threading
+    import torch
+    rng = np.random.default_rng(77 + mode)
+    graphs = [er(n, 0.4, 3 * n) for n in (15, 7)]
+    beta, gamma = rng.uniform(-4, 4, size=(2, 6, len(graphs), 3))
+    batches = [E.QAOABatch(graphs, 3, mode=mode) for _ in range(6)]
+    got, gate = [None] * 6, threading.Barrier(6)
+    torch.cuda.synchronize()
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            gate.wait()
+            got[i] = batches[i].evaluate(beta[i], gamma[i])
+            torch.cuda.current_stream().synchronize()
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i, b in enumerate(batches):
+        b.check()
+        parts = [x.cpu().numpy().copy() for x in got[i] if x is not None]
+        again = [x.cpu().numpy() for x in b.evaluate(beta[i], gamma[i]) if x is not None]
+        for x, y in zip(parts, again):
+            assert np.array_equal(x, y)
