@@ -485,3 +485,31 @@ def test_batches_of_several_threads(E, mode):
         again = [x.cpu().numpy() for x in b.evaluate(beta[i], gamma[i]) if x is not None]
         for x, y in zip(parts, again):
             assert np.array_equal(x, y)
+
+
+def test_two_launches_that_fill_the_device(E):
+    """Two batches of more workgroups than run at once, on two streams: where
+    each holds a part of the CUs, either still finishes, with the bits of a
+    launch of its own."""
+    import torch
+    graphs = [er(n, 0.3, n + i) for i, n in enumerate([16, 17] * 24)]
+    rng = np.random.default_rng(5)
+    angles = rng.uniform(-3, 3, size=(2, 2, len(graphs), 4))
+    batches = [E.QAOABatch(graphs, 4, mode=E.MODE_BACKWARD) for _ in range(2)]
+    want = []
+    for b, (beta, gamma) in zip(batches, angles):
+        assert b._args.max_items_per_k >= 512
+        b.evaluate(beta, gamma)
+        want.append(b.out.clone())
+    streams = [torch.cuda.Stream() for _ in batches]
+    for _ in range(4):
+        for b in batches:
+            b.out.zero_()
+        torch.cuda.synchronize()
+        for b, st in zip(batches, streams):
+            with torch.cuda.stream(st):
+                for _ in range(3):
+                    b.launch()
+        for b, w in zip(batches, want):
+            b.check()
+            assert torch.equal(b.out, w)
