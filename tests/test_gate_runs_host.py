@@ -124,3 +124,40 @@ def test_class_pickled_without_a_record_slot_loads():
     old = type(kind).__new__(type(kind))
     old.__setstate__((None, {n: getattr(kind, n) for n in kind.__slots__ if n != '_record'}))
     assert old.record()[1].k == 2
+
+
+@pytest.mark.parametrize("k", [0, 1, 2, 3, 4, 5, 6])
+def test_gate_classes_by_width(k):
+    # read as lists up to 3 qubits, by numpy above; dense from 6 on
+    rng = np.random.default_rng(k)
+    dim = 2 ** k
+    phases = np.exp(1j * rng.uniform(0, 6, dim))
+    perm = np.roll(np.arange(dim), 1)
+    zero_row = np.diag(phases)
+    zero_row[0, 0] = 0
+    twice = np.eye(dim)[np.zeros(dim, dtype=int)]          # one entry a row, no permutation
+    moves = dim > 1
+    for m, kind, src, phase in [
+            (np.diag(phases), 'diagonal', None, None), (zero_row, 'diagonal', None, None),
+            (np.eye(dim)[perm], 'monomial' if moves else 'diagonal', perm, None),
+            (phases[:, None] * np.eye(dim)[perm], 'monomial' if moves else 'diagonal', perm, phases),
+            (twice, 'dense' if moves else 'diagonal', None, None),
+            (np.full((dim, dim), np.nan), 'dense' if moves else 'diagonal', None, None)]:
+        got = ops.bk.classify(m)
+        assert got.kind == ('dense' if k > 5 else kind)
+        if got.kind == 'diagonal':
+            assert np.array_equal(got.diag, np.diag(m).astype(complex), equal_nan=True)
+        if got.kind == 'monomial':
+            assert got.src.dtype == np.int32 and np.array_equal(got.src, src)
+            assert got.phase is None if phase is None else np.array_equal(got.phase, phase)
+
+
+def test_classes_of_wide_gates_cost_little_more():
+    # a 5-qubit matrix has 16 times the entries of a 3-qubit one; read entry by
+    # entry it took 8 times as long, by numpy twice
+    import timeit
+    cost = []
+    for k in (3, 5):
+        m = np.linalg.qr(np.random.default_rng(k).normal(size=(2 ** k, 2 ** k)))[0].astype(complex)
+        cost.append(min(timeit.repeat(lambda: ops.bk.classify(m), number=200, repeat=5)))
+    assert cost[1] <= 4 * cost[0]
