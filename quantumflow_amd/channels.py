@@ -14,6 +14,7 @@ products, identity, diagonal, trace, partial trace and the weighted sums
 of wider Kraus channels run in csrc/density.hip.
 """
 
+from functools import partial
 from typing import Sequence, Union
 
 import numpy as np
@@ -176,42 +177,44 @@ def gate_evolve(gate: Gate, rho: Density) -> Density:
     on both sets of axes, fits a single gate kernel (dense with 2K <= 3,
     diagonal or monomial with 2K <= 5: every 1-qubit gate, CNOT, CZ, SWAP,
     ISWAP, ...) the map is one pass over the density; otherwise two."""
-    N = rho.qubit_nb
-    idx = [rho.qubits.index(q) for q in gate.qubits]
-    k = len(idx)
+    return evolve_by(_gate_kinds(gate), gate.qubits, rho)
+
+
+def _gate_kinds(gate):
     m = gate.matrix
-    cols = [N + i for i in idx]
     kind = _one_pass_kind(m)
     if kind is not None:
-        t = bk.tensormul(kind, rho.tensor, idx + cols)
-        return Density(t, rho.qubits, rho._memory)
-    t = bk.tensormul(m.reshape([2] * (2 * k)), rho.tensor, idx)
-    t = bk.tensormul(np.conj(m).reshape([2] * (2 * k)), t, cols)
+        return [(kind, 'both')]
+    return [(gate.kind, 'rows'), (bk.classify(np.conj(m)), 'cols')]
+
+
+def evolve_by(kinds, qubits, rho: Density) -> Density:
+    """The gates ``kinds`` of evolve_kinds on a density, one pass each."""
+    N = rho.qubit_nb
+    rows = [rho.qubits.index(q) for q in qubits]
+    cols = [N + i for i in rows]
+    t = rho.tensor
+    for kind, where in kinds:
+        t = bk.tensormul(kind, t, rows + cols if where == 'both' else
+                         (rows if where == 'rows' else cols))
     return Density(t, rho.qubits, rho._memory)
 
 
 def evolve_kinds(elem):
-    """How the gate-list kernel evolves a density by ``elem``: [(kernel class,
-    axes)] with axes 'rows', 'cols' or 'both' (rows then columns) of the
-    element's qubits, the gates that gate_evolve, Kraus.evolve and
-    Channel.evolve apply one pass each; None where it does not take them or
-    the element's evolve is its own."""
+    """How ``elem`` evolves a density: [(kernel class, axes)], gates that the
+    gate-list kernel takes on the row axes ('rows'), column axes ('cols') or
+    both of the element's qubits; or a function of the density, where it does
+    not take them or the element's evolve is its own."""
     method = getattr(type(elem), 'evolve', None)
-    if isinstance(elem, Gate) and method is Gate.evolve:
-        if elem.qubit_nb > 3:
-            return None
-        m = elem.matrix
-        kind = _one_pass_kind(m)
-        if kind is not None:
-            return [(kind, 'both')]
-        return [(elem.kind, 'rows'), (bk.classify(np.conj(m)), 'cols')]
-    if isinstance(elem, Kraus) and method is Kraus.evolve:
+    if method is Gate.evolve and elem.qubit_nb <= 3:
+        return _gate_kinds(elem)
+    if method is Kraus.evolve:
         kind = elem._one_pass_kind()
-        return None if kind is None else [(kind, 'both')]
-    if isinstance(elem, Channel) and method is Channel.evolve:
-        kind = bk.classify(elem._mat)
-        return [(kind, 'both')] if kind.listable else None
-    return None
+        return elem._evolve_terms if kind is None else [(kind, 'both')]
+    if method is Channel.evolve:
+        kinds = [(bk.classify(elem._mat), 'both')]
+        return kinds if kinds[0][0].listable else partial(evolve_by, kinds, elem.qubits)
+    return elem.evolve
 
 
 class Channel(Operation):
@@ -334,11 +337,7 @@ class Channel(Operation):
     def evolve(self, rho: Density) -> Density:
         """The superoperator on the channel's row and column axes of the
         density, one gate-kernel pass (ops.py:354-363)."""
-        N = rho.qubit_nb
-        idx = [rho.qubits.index(q) for q in self.qubits]
-        kind = bk.classify(self._mat)
-        t = bk.tensormul(kind, rho.tensor, idx + [N + i for i in idx])
-        return Density(t, rho.qubits, rho._memory)
+        return evolve_by([(bk.classify(self._mat), 'both')], self.qubits, rho)
 
     def __add__(self, other) -> 'Channel':
         if isinstance(other, Channel):
@@ -420,10 +419,10 @@ class Kraus(Operation):
         accumulated by weighted sums."""
         kind = self._one_pass_kind()
         if kind is not None:
-            N = rho.qubit_nb
-            idx = [rho.qubits.index(q) for q in self.qubits]
-            t = bk.tensormul(kind, rho.tensor, idx + [N + i for i in idx])
-            return Density(t, rho.qubits, rho._memory)
+            return evolve_by([(kind, 'both')], self.qubits, rho)
+        return self._evolve_terms(rho)
+
+    def _evolve_terms(self, rho: Density) -> Density:
         out = torch.zeros(4 ** rho.qubit_nb, dtype=torch.complex128, device=bk.DEVICE)
         for op, w in zip(self.operators, self.weights):
             term = bk.as_device(op.evolve(rho).tensor)

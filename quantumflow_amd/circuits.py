@@ -15,6 +15,7 @@ from typing import Dict, Iterable, Iterator, Sequence, Type
 
 from . import backend as bk
 from . import config
+from .channels import Density, evolve_by, evolve_kinds
 from .gates import control_gate, identity_gate
 from .ops import Gate, Operation
 from .qubits import Qubit, Qubits
@@ -40,22 +41,21 @@ def _listed(elem, method):
 
 
 def _runs(elements, item):
-    """Split ``elements`` into maximal runs: yields (list of (elem, item(elem))
-    pairs, None) for runs of at least two elements with an item, else
-    (None, elem)."""
+    """Split ``elements`` into maximal runs for the gate-list kernel: yields
+    lists of (elem, item(elem)) pairs.  An element whose item is None or a
+    function is a list of its own."""
     run = []
-    for elem in chain(elements, [None]):
-        it = item(elem) if elem is not None else None
-        if it is not None:
+    for elem in elements:
+        it = item(elem)
+        if it is not None and not callable(it):
             run.append((elem, it))
             continue
-        if len(run) > 1:
-            yield run, None
-        elif run:
-            yield None, run[0][0]
-        run = []
-        if elem is not None:
-            yield None, elem
+        if run:
+            yield run
+            run = []
+        yield [(elem, it)]
+    if run:
+        yield run
 
 
 def _bits_of(qubits, axes):
@@ -131,13 +131,15 @@ class Circuit(Operation):
         default |0...0><0...0| on the circuit's qubits."""
         if rho is None:
             rho = zero_state(qubits=self.qubits).asdensity()
-        from .channels import evolve_kinds, Density
-        for run, elem in _runs(self.elements, evolve_kinds):
-            if run is None:
-                rho = elem.evolve(rho)
+        if len(self.elements) == 1:
+            return self.elements[0].evolve(rho)
+        for run in _runs(self.elements, evolve_kinds):
+            if len(run) == 1:
+                elem, how = run[0]
+                rho = how(rho) if callable(how) else evolve_by(how, elem.qubits, rho)
                 continue
-            # each element's kernel gates act on its qubits' row axes, then
-            # (or also) on their column axes
+            # each element's kernel gates act on its qubits' row axes, their
+            # column axes or both
             n = rho.qubit_nb
             bit_of = _bits_of(rho.qubits, 2 * n)
             kinds, bits = [], []
@@ -161,6 +163,8 @@ class Circuit(Operation):
         if ket is None:
             ket = zero_state(qubits=self.qubits)
         if fused is None:
+            if len(self.elements) == 1:
+                return self.elements[0].run(ket)
             if config.FUSION and 0 < ket.qubit_nb < FUSED_MIN_QUBITS:
                 return self._run_small(ket)
             fused = config.FUSION and ket.qubit_nb >= FUSED_MIN_QUBITS
@@ -192,9 +196,9 @@ class Circuit(Operation):
                     yield from flat(elem)
                 else:
                     yield elem
-        for run, elem in _runs(flat(self), lambda e: _listed(e, 'run')):
-            if run is None:
-                ket = elem.run(ket)
+        for run in _runs(flat(self), lambda e: _listed(e, 'run')):
+            if len(run) == 1:
+                ket = run[0][0].run(ket)
                 continue
             # a density's gates act on its row axes, as Gate.run's do
             bit_of = _bits_of(ket.qubits, bk.rank(ket.tensor))
@@ -213,9 +217,9 @@ class Circuit(Operation):
             if isinstance(elem, Gate) and type(elem).__matmul__ is Gate.__matmul__:
                 return _listed(elem, 'asgate')
             return None                         # nested circuits among them
-        for run, elem in _runs(self.elements, item):
-            if run is None:
-                gate = elem.asgate() @ (identity_gate(qubits) if gate is None else gate)
+        for run in _runs(self.elements, item):
+            if len(run) == 1:
+                gate = run[0][0].asgate() @ (identity_gate(qubits) if gate is None else gate)
                 continue
             n = len(qubits)
             bit_of = _bits_of(qubits, 2 * n)
