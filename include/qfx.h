@@ -441,8 +441,10 @@ typedef struct {
   int32_t ninst, nk, width, mode, block, max_items_per_k;
   int32_t tile_bits;      /* largest pass tile, at most 13 forward and 12
                              backward; 0: 13 in either (13-bit backward tiles
-                             take a CU each, all others half of one).  Must be
-                             what qfx_qaoa_check accepted the program with. */
+                             take a CU each, as do 12-bit ones with weighted
+                             instances or without `tables`; all others half
+                             of one).  Must be what qfx_qaoa_check accepted
+                             the program with. */
   int32_t pad;
   void* timing;           /* NULL, or uint64 [timing_len]: per global pass k
                              and workgroup b, entries 2 (k grid + b) and +1

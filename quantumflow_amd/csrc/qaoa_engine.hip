@@ -857,8 +857,11 @@ __device__ bool grid_barrier(unsigned* counter, unsigned target, int* err,
 // not started), so the first unfinished one can always go on.  Else:
 // items in turn, and a grid barrier with a cache flush after each pass.  WTD:
 // the launch may hold weighted instances, whose phases are made in place.
-// WIDE: 13-bit tiles of psi and lambda, 256 registers a lane, one workgroup a
-// CU; all else fits 128 registers and two.
+// WIDE: 256 registers a lane and one workgroup a CU, for 13-bit tiles of psi
+// and lambda, and for 12-bit ones where phases are made in place (in 128
+// registers 81 were spilled, into the sincos loop: 8 weighted instances of 12
+// qubits and 4 layers 165 us, now 86; 512 of 14 978, now 571); all else fits 128
+// registers and two.
 //
 // What bounds it: with its tile in registers an item of 13 bits backward takes
 // 25 us a layer on the way there and 45 us back on its CU, of which the mixer's
@@ -921,7 +924,7 @@ void qaoa_kernel(
       };
       switch (ps.T) {
         case 13: if constexpr (!BWD || WIDE) run(std::integral_constant<int, 4>{}); break;
-        case 12: run(std::integral_constant<int, 3>{}); break;
+        case 12: if constexpr (!BWD || WIDE || !WTD) run(std::integral_constant<int, 3>{}); break;
         case 11: run(std::integral_constant<int, 2>{}); break;
         case 10: run(std::integral_constant<int, 1>{}); break;
         default: run(std::integral_constant<int, 0>{}); break;
@@ -1191,7 +1194,9 @@ int qfx_qaoa_run(void* stream, const qfx_qaoa_args* args) {
   hipStream_t s = qfx::as_stream(stream);
   // programs without cut values hold no weighted instance
   const bool flow = a.tables && a.table_off && a.item_need, weighted = a.val_pool;
-  const bool wide = a.tile_bits == 0;
+  // in-place phases (weighted instances; every launch with barriers) leave no
+  // registers for 12-bit tiles at two workgroups a CU
+  const bool wide = a.tile_bits == 0 || (a.tile_bits == 12 && (!flow || weighted));
   if (a.mode == QFX_QAOA_BACKWARD && wide)
     return !flow      ? launch_qaoa<true, false, true, true>(s, a)
            : weighted ? launch_qaoa<true, true, true, true>(s, a)

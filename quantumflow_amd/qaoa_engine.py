@@ -133,7 +133,8 @@ def batch_bits(ns, mode, T):
     layers: 128 instances of 13 qubits 243 / 207 us, 16 of 18 609 / 594, 8 of
     19 835 / 635, 1 of 22 977 / 681, 1 of 23 2980 / 1475, 1 of 24 6468 / 3347;
     but 4 of 19 371 / 444, 1 of 20 286 / 411, 1 of 21 413 / 526, and 64 of 16
-    414 / 499."""
+    414 / 499; at 4 layers 512 of 14 qubits 336 / 956, 512 of 15 688 / 960, 64
+    of 17 352 / 481."""
     if mode == MODE_BACKWARD and T == 12:
         gain = [n == 13 or n >= 18 for n in ns]
         if sum(2 ** max(n - 14, 0) for n, g in zip(ns, gain) if g) >= 192:
@@ -334,7 +335,12 @@ class QAOABatch:
         cut_jobs = []
         arrays = [graph_arrays(g) for g in self.graphs]
         self.n = [x[0] for x in arrays]
-        self._bits = batch_bits(self.n, mode, T)
+        # weighted instances below 23 qubits keep T: their phases are made in
+        # place, and 13-bit tiles leave no registers for that.  12 / 13 bits, 4
+        # layers: 64 of 18 qubits 1407 / 2406 us, 16 of 20 1400 / 2463, 1 of 22
+        # 554 / 704, 1 of 23 1521 / 1392
+        self._bits = [T if x[3] and x[0] < 23 else b
+                      for x, b in zip(arrays, batch_bits(self.n, mode, T))]
         for i, (n, edges, w, weighted) in enumerate(arrays):
             width = self._bits[i]
             mir = bool(mirror) and use_mirror(n, width)
