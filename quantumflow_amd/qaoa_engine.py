@@ -292,6 +292,21 @@ def graph_arrays(graph):
     return n, np.array(edges, dtype=np.int32).reshape(-1, 2), w, weighted
 
 
+def upload(arrays):
+    """Host arrays (ctypes or numpy) in one device tensor, by one copy: the
+    tensor and each array's address, 16-byte aligned."""
+    off, total = [], 0
+    for a in arrays:
+        off.append(total)
+        total += -(-memoryview(a).nbytes // 16) * 16
+    host = np.zeros(total, np.uint8)
+    for a, o in zip(arrays, off):
+        part = np.frombuffer(a, np.uint8)
+        host[o:o + len(part)] = part
+    dev = torch.from_numpy(host).to(bk.DEVICE)
+    return dev, [dev.data_ptr() + o for o in off]
+
+
 class QAOABatch:
     """A fixed batch of MaxCut instances compiled for the GPU engine.
 
@@ -413,6 +428,7 @@ class QAOABatch:
                     items.append(it)
                     need.append(q * tiles)
                 kstart.append(len(items))
+        self._kstart = kstart
         self.nk = len(kstart) - 1
         self.nitems = len(items)
         psi_len = max(psi_len, single_max)
@@ -433,12 +449,14 @@ class QAOABatch:
                                          tile_bits),
                       'qfx_qaoa_check')
 
-        def up(arr):
-            return torch.frombuffer(bytearray(bytes(arr)), dtype=torch.uint8).to(dev)
-        self._insts = up(insts)
-        self._passes = up(passes_arr)
-        self._items = up(items_arr)
-        self._kstart = torch.tensor(kstart, dtype=torch.int32, device=dev)
+        # every launch's counters, mixers and cost phases (qfx_qaoa_args.tables)
+        head = TABLE_HEAD + ninst
+        sizes = [p * (MIXER + (0 if i.weighted else i.nedges + 1)) for i in insts]
+        table_off = head + np.concatenate([[0], np.cumsum(sizes)[:-1]])
+        self._tables = torch.empty(head + sum(sizes), dtype=torch.complex128, device=dev)
+        # the program in one copy (six took 55 us of a 9-qubit batch's 275)
+        self._program, at = upload([insts, passes_arr, items_arr, ks,
+                                    table_off.astype(np.int64), np.array(need, np.int32)])
         self.psi_pool = torch.empty(psi_len, dtype=torch.complex128, device=dev)
         self.lam_pool = torch.empty(lam_len if mode == MODE_BACKWARD else 1,
                                     dtype=torch.complex128, device=dev)
@@ -448,12 +466,6 @@ class QAOABatch:
         self.out = torch.zeros(ninst * self.width, dtype=torch.float64, device=dev)
         self.sync = torch.zeros(4, dtype=torch.int32, device=dev)
         self.angles = torch.zeros(ninst * 2 * p, dtype=torch.float64, device=dev)
-        # every launch's counters, mixers and cost phases (qfx_qaoa_args.tables)
-        head = TABLE_HEAD + ninst
-        sizes = [p * (MIXER + (0 if i.weighted else i.nedges + 1)) for i in insts]
-        self._table_off = torch.tensor(head + np.concatenate([[0], np.cumsum(sizes)[:-1]]),
-                                       dtype=torch.int64, device=dev)
-        self._tables = torch.empty(head + sum(sizes), dtype=torch.complex128, device=dev)
         # cut tables on the GPU
         s = bk.stream_handle()
         for (n, edges, w, weighted, off) in cut_jobs:
@@ -472,9 +484,8 @@ class QAOABatch:
                 float((tab.to(torch.int32) & 0xFFFF).max().item())
         self._args = QaoaArgs()
         a = self._args
-        a.insts, a.passes, a.items = self._insts.data_ptr(), self._passes.data_ptr(), \
-            self._items.data_ptr()
-        a.kstart, a.angles = self._kstart.data_ptr(), self.angles.data_ptr()
+        a.insts, a.passes, a.items, a.kstart = at[:4]
+        a.angles = self.angles.data_ptr()
         a.psi_pool, a.lam_pool = self.psi_pool.data_ptr(), self.lam_pool.data_ptr()
         a.cnt_pool = self.cnt_pool.data_ptr()
         a.val_pool = self.val_pool.data_ptr() if val_len else None
@@ -483,10 +494,8 @@ class QAOABatch:
         a.ninst, a.nk, a.width, a.mode, a.block = ninst, self.nk, self.width, mode, block
         a.max_items_per_k = max(kstart[k + 1] - kstart[k] for k in range(self.nk))
         a.tile_bits = tile_bits
-        self._need = torch.tensor(need, dtype=torch.int32, device=dev)
         if flow:
-            a.tables, a.table_off = self._tables.data_ptr(), self._table_off.data_ptr()
-            a.item_need = self._need.data_ptr()
+            a.tables, a.table_off, a.item_need = self._tables.data_ptr(), at[4], at[5]
         self._graph = None
 
     def algorithmic_bytes(self):
@@ -568,7 +577,7 @@ class QAOABatch:
         grid = int(np.count_nonzero(flat)) // (2 * self.nk)
         st = flat[:2 * self.nk * grid].reshape(self.nk, grid, 2)
         us = 1e3 / khz
-        ks = self._kstart.cpu().numpy()
+        ks = self._kstart
         out = []
         for k in range(self.nk):
             s0, s1 = st[k, :, 0], st[k, :, 1]

@@ -323,3 +323,19 @@ def test_instance_groups_hold_every_instance_once(limit):
         assert len(groups) == 1
     assert E.instance_groups([], limit) == []
     assert E.instance_groups([2 ** 32], limit) == [[0]]
+
+
+def test_upload_holds_every_array(monkeypatch):
+    import ctypes
+    monkeypatch.setattr(E.bk, 'DEVICE', 'cpu')
+    insts = (E.QaoaInst * 3)()
+    insts[2].n = 7
+    arrays = [insts, (ctypes.c_int * 3)(0, 5, 9), np.array([4, 2 ** 40]),
+              np.array([7], np.int32), np.arange(33, dtype=np.int32)]
+    dev, at = E.upload(arrays)
+    end = dev.data_ptr()
+    for a, p in zip(arrays, at):
+        assert p % 16 == dev.data_ptr() % 16 and p >= end
+        end = p + memoryview(a).nbytes
+        assert ctypes.string_at(p, memoryview(a).nbytes) == memoryview(a).tobytes()
+    assert end <= dev.data_ptr() + dev.numel()
