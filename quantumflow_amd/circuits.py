@@ -42,20 +42,40 @@ def _listed(elem, method):
 
 def _runs(elements, item):
     """Split ``elements`` into maximal runs for the gate-list kernel: yields
-    lists of (elem, item(elem)) pairs.  An element whose item is None or a
-    function is a list of its own."""
+    lists of (elem, item(elem)) pairs.  An element without an item is a list of
+    its own."""
     run = []
     for elem in elements:
         it = item(elem)
-        if it is not None and not callable(it):
+        if it is not None:
             run.append((elem, it))
             continue
         if run:
             yield run
             run = []
-        yield [(elem, it)]
+        yield [(elem, None)]
     if run:
         yield run
+
+
+def _evolve_run(run, rho):
+    """A density evolved by (element, kinds of evolve_kinds) pairs: each
+    element's kernel gates act on its qubits' row axes, their column axes or
+    both."""
+    if len(run) < 2:
+        for elem, gates in run:
+            rho = evolve_by(gates, elem.qubits, rho)
+        return rho
+    n = rho.qubit_nb
+    bit_of = _bits_of(rho.qubits, 2 * n)
+    kinds, bits = [], []
+    for elem, gates in run:
+        rows = _lookup(bit_of, elem.qubits)
+        cols = [b - n for b in rows]
+        for kind, where in gates:
+            kinds.append(kind)
+            bits += rows + cols if where == 'both' else (rows if where == 'rows' else cols)
+    return Density(bk.apply_gates(rho.tensor, kinds, bits), rho.qubits, rho._memory)
 
 
 def _bits_of(qubits, axes):
@@ -133,25 +153,15 @@ class Circuit(Operation):
             rho = zero_state(qubits=self.qubits).asdensity()
         if len(self.elements) == 1:
             return self.elements[0].evolve(rho)
-        for run in _runs(self.elements, evolve_kinds):
-            if len(run) == 1:
-                elem, how = run[0]
-                rho = how(rho) if callable(how) else evolve_by(how, elem.qubits, rho)
-                continue
-            # each element's kernel gates act on its qubits' row axes, their
-            # column axes or both
-            n = rho.qubit_nb
-            bit_of = _bits_of(rho.qubits, 2 * n)
-            kinds, bits = [], []
-            for e, gates in run:
-                rows = _lookup(bit_of, e.qubits)
-                cols = [b - n for b in rows]
-                for kind, where in gates:
-                    kinds.append(kind)
-                    bits += rows + cols if where == 'both' else \
-                        (rows if where == 'rows' else cols)
-            rho = Density(bk.apply_gates(rho.tensor, kinds, bits), rho.qubits, rho._memory)
-        return rho
+        run = []
+        for elem in self.elements:
+            how = evolve_kinds(elem)
+            if callable(how):
+                rho = how(_evolve_run(run, rho))
+                run = []
+            else:
+                run.append((elem, how))
+        return _evolve_run(run, rho)
 
     def run(self, ket: State = None, fused: bool = None) -> State:
         """Apply the circuit to ``ket`` (default |0...0> on the sorted
@@ -214,9 +224,10 @@ class Circuit(Operation):
         gate = None
 
         def item(elem):
-            if isinstance(elem, Gate) and type(elem).__matmul__ is Gate.__matmul__:
+            # nested circuits, among others, have no __matmul__
+            if getattr(type(elem), '__matmul__', None) is Gate.__matmul__:
                 return _listed(elem, 'asgate')
-            return None                         # nested circuits among them
+            return None
         for run in _runs(self.elements, item):
             if len(run) == 1:
                 gate = run[0][0].asgate() @ (identity_gate(qubits) if gate is None else gate)

@@ -454,7 +454,8 @@ class QAOABatch:
         sizes = [p * (MIXER + (0 if i.weighted else i.nedges + 1)) for i in insts]
         table_off = head + np.concatenate([[0], np.cumsum(sizes)[:-1]])
         self._tables = torch.empty(head + sum(sizes), dtype=torch.complex128, device=dev)
-        # the program in one copy (six took 55 us of a 9-qubit batch's 275)
+        # the program in one copy: 1 instance of 9 qubits is built in 189 us, with
+        # six copies in 275
         self._program, at = upload([insts, passes_arr, items_arr, ks,
                                     table_off.astype(np.int64), np.array(need, np.int32)])
         self.psi_pool = torch.empty(psi_len, dtype=torch.complex128, device=dev)
