@@ -437,7 +437,7 @@ typedef struct {
                              error flag, sticky error flag.  The owner zeroes
                              all three before the first launch; a launch
                              resets the first two and leaves the third, which
-                             any grid-barrier timeout sets. */
+                             any wait that times out sets. */
   int32_t ninst, nk, width, mode, block, max_items_per_k;
   int32_t tile_bits;      /* largest pass tile, at most 13 forward and 12
                              backward; 0: 13 in either (13-bit backward tiles

@@ -289,7 +289,7 @@ __device__ __forceinline__ void list_rows(int T, int tid, const u32x4 w, const v
 // ops are staged behind the tile once per workgroup: fetched from the argument
 // memory as they came, each waited about a microsecond (40 us instead of 20
 // for 28 gates at 9 qubits).
-// 360 gates, 12 qubits: 243 us in 6 launches (one launch a gate: 7.4 ms, of
+// 360 gates, 12 qubits: 242 us in 5 launches (one launch a gate: 7.4 ms, of
 // which 1.1 ms on the GPU).  24 index bits: 100 us a pass and 13-16 us a gate,
 // where a gate of its own takes 90-100 us.
 template <int BS>

@@ -49,9 +49,9 @@ enum Stage : int {
   ST_MAKE_LAMBDA = 5,  // lambda <- C psi
   ST_RX_ADJ = 6,       // grad_beta += Im sum <lam|X_j|psi>; RX(-beta) on psi, lam
   ST_COST_ADJ = 7,     // grad_gamma += 2 Im <lam|C|psi> - W Im <lam|psi>; conj phases
-  ST_COST_RX = 8,      // ST_COST then ST_RX of the same layer (phases in one RX chunk)
-  ST_RX_LOAD = 10,     // ST_RX applied while the tile is loaded (first stage)
-  ST_RX_STORE = 11,    // ST_RX applied while the tile is stored (last stage)
+  ST_COST_RX = 8,      // ST_COST then ST_RX of the same layer
+  ST_RX_LOAD = 10,     // ST_RX as the first stage of a pass that loads
+  ST_RX_STORE = 11,    // ST_RX as the last stage of a pass that stores
 };
 
 enum PassFlags : int { PF_LOAD_PSI = 1, PF_LOAD_LAM = 2, PF_STORE_PSI = 4, PF_STORE_LAM = 8 };
@@ -60,7 +60,7 @@ constexpr int kMaxT = 13;
 constexpr int kMaxPLayers = QFX_QAOA_MAX_LAYERS;
 constexpr int kAccum = 1 + 2 * kMaxPLayers;  // value, d/dbeta, d/dgamma
 constexpr int kMaxEdgesTab = 512;  // cut counts 0..kMaxEdgesTab-1 tabulated
-// A grid barrier gives up after kBarrierSeconds of wall-clock time.  One
+// A wait gives up after kBarrierSeconds of wall-clock time.  One
 // phase of the largest program qfx_qaoa_check accepts (n <= 30: a 16 GiB
 // state read and written once) streams in well under 0.1 s, so a timeout
 // means workgroups that never arrive, not a slow phase.
@@ -510,6 +510,14 @@ __device__ __forceinline__ bool is_mixer(int type) {
 // go to memory at agent scope (sc1: past this XCD's L2 where another XCD may
 // hold newer data); 16 bytes a lane as the buffer forms take, which is why the
 // pool of one instance stays under 2^31 bytes.
+// No release or acquire fence is needed beside them: at agent scope these
+// write the L2 back and drop its lines, for accesses that stop there, and the
+// pools' do not.  What is needed is order.  A workgroup's stores have reached
+// memory before it counts its item (stores_done, then the barrier, then one
+// lane's atomic, itself at agent scope); a workgroup loads only after the count
+// was seen (one lane polls, then the barrier, which the compiler moves no
+// access across).  The pools are all that passes between workgroups of a
+// launch: tables come from the kernel before, partial sums go to the one after.
 template <bool FLOW>
 struct Pool;
 

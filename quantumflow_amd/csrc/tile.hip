@@ -39,11 +39,11 @@ constexpr int kMaxStaged = 768;
 
 // Where a pass loads and stores: from `from`, to `state`.  The two are one
 // (a pass in place) or do not overlap: the first pass of a circuit reads the
-// caller's state: with a copy of it 36.4 and not 34.4 ms for 728 gates on 28
-// qubits, 253 and not 217 us for 520 on 20.  A tile is stored to the indices it was loaded from, possibly
-// with its tile bits permuted (tile bit j is stored to index bit d[j], a
-// permutation of s[0..T-1]: the qubit relabelling of the SWAP gates the pass
-// absorbed).
+// caller's state (with a copy of it 36.4 and not 34.4 ms for 739 gates on 28
+// qubits, 253 and not 217 us for 551 on 20).  A tile is stored to the indices
+// it was loaded from, possibly with its tile bits permuted (tile bit j is
+// stored to index bit d[j], a permutation of s[0..T-1]: the qubit relabelling
+// of the SWAP gates the pass absorbed).
 struct TilePos {
   int s[QFX_MAX_QUBITS];   // tile bit positions, ascending (where tile bit j loads from)
   int d[QFX_MAX_QUBITS];   // where tile bit j is stored

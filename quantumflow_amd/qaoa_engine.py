@@ -44,9 +44,12 @@ MAX_STAGES = 40
 LOW_BITS = 3
 FLOW_KEPT = 2 ** 27       # kept amplitudes that qfx_qaoa_args.item_need allows
 # State of the instances whose passes are listed together: their passes follow
-# each other while it is still in the 256 MiB cache beside the cut tables.  104
-# values of 10 to 22 qubits (512 MiB of state): 64 MiB 1466 us, 96 1386, 128
-# 1204, 192 1196, 256 1268, all at once 1309; smaller groups run out of items.
+# each other while it is still in the 256 MiB cache beside the cut tables; smaller
+# groups run out of items.  64 / 96 / 128 / 192 / 256 MiB / all at once: 104
+# values of 10 to 22 qubits 1287 / 1095 / 899 / 899 / 946 / 1010 us, 512 of them
+# 7985 / 5835 / 5279 / 5064 / 5222 / 5615, 64 values of 20 qubits 2034 / 1221 /
+# 945 / 928 / 958 / 1021, their gradients 4734 / 3981 / 4020 / 3993 / 4234 / 4547,
+# 65 gradients of 16 to 24 qubits within 0.4% from 128 MiB on.
 GROUP_BYTES = 192 * 2 ** 20
 TABLE_HEAD, MIXER = 32, 8  # entries of qfx_qaoa_args.tables
 
@@ -546,8 +549,8 @@ class QAOABatch:
         self._graph.replay()
 
     def check(self):
-        """Synchronise and raise if a grid barrier timed out in any launch
-        since the batch was built (the kernel's error word is sticky: a
+        """Synchronise and raise if a wait for items or a grid barrier timed out
+        in any launch since the batch was built (the kernel's error word is sticky: a
         later launch does not clear it)."""
         failed = ctypes.c_int(0)
         torch.cuda.synchronize()
@@ -593,7 +596,7 @@ class QAOABatch:
     def evaluate(self, beta, gamma, graph=False):
         """(values [ninst], grads [ninst, 2p] or None) as device tensors.
         The launch is asynchronous: ``check()`` (which synchronises) raises
-        if any launch since the batch was built hit a barrier timeout, so
+        if a wait timed out in any launch since the batch was built, so
         one call after a run of evaluations covers all of them."""
         self.set_angles(beta, gamma)
         if graph:
@@ -610,7 +613,8 @@ def raise_if_failed(flag):
     """The engine's status word: nonzero means a wait for other items gave up, and
     the values and gradients of that launch are partial."""
     if flag:
-        raise RuntimeError('qaoa engine: grid barrier timed out; results are partial')
+        raise RuntimeError('qaoa engine: a wait for items or a grid barrier timed out; '
+                           'results are partial')
 
 
 class QAOAExpectation(torch.autograd.Function):
